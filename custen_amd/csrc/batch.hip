@@ -2,9 +2,9 @@
 // together: one launch per step covers every strip of every grid (the
 // workgroup finds its grid by binary search over the strip prefix sums), and
 // a whole multi-step run is captured once into a HIP graph and replayed.
-// With the band walker selected, a step is two launches: the band walker over
-// the interior 128-column strips of every grid (one wave per band, found the
-// same way), then the strip kernel over the remaining edge strips.  The
+// With the band walker selected, a step walks every grid that is at least a
+// strip wide and a chunk high (one wave per band, found the same way); a
+// second launch runs the strip kernel over the smaller grids, if any.  The
 // per-grid launch loop (one launch per grid per step) is kept as the baseline
 // mode.  Per grid the arithmetic is the single-grid kernels' (stencil_body.h,
 // stencil_band.h), so results are bit-identical to cuStenCompute2DXYp.
@@ -35,11 +35,11 @@ struct BatchDev {
     int nx, ny;
     int stripBase;  // first strip id of this grid (strip kernel over all strips)
     int vec;        // rows pair-aligned
-    // band-walker split: strips [0, nBandTx) are walked by bands, strips
-    // [nBandTx, tilesX) run the strip kernel
+    // with the band walker: a grid it applies to is walked as a whole, the
+    // others' strips run the strip kernel
+    int walked;
     int bandBase;   // first band item (wave) of this grid
-    int nBandTx;
-    int edgeBase;   // first edge-strip item of this grid
+    int restBase;   // first strip item of this grid, if it is not walked
 };
 
 namespace dev {
@@ -86,8 +86,8 @@ __device__ __forceinline__ StencilLaunch gridLaunch(const BatchDev& G, int parit
     return a;
 }
 
-// Strip kernel over every strip of every grid (edges = 0) or over the edge
-// strips [nBandTx, tilesX) of every grid (edges = 1).
+// Strip kernel over every strip of every grid (rest = 0) or over those of the
+// grids that are not walked (rest = 1).
 // itemGrid[item] is the grid that owns the item (built on the host with the
 // item tables, so a workgroup finds its grid with one load).
 template <typename T, int H, int V, int RPW>
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restri
                                                         const int* __restrict__ itemGrid,
                                                         int firstItem, int parity,
                                                         const double* __restrict__ weights, int L,
-                                                        int Tt, int chunks, int edges)
+                                                        int Tt, int chunks, int rest)
 {
     __shared__ __attribute__((aligned(16))) T tile[(kWaves * RPW + V - 1) * ldsRowLength(H)];
     T w[H * V];
@@ -106,14 +106,13 @@ __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restri
     const StencilLaunch a = gridLaunch(G, parity, sizeof(T) == 8 ? Dtype::F64 : Dtype::F32,
                                        weights, H, L, V, Tt, RPW, chunks);
     const int tilesX = (G.nx + kTW - 1) / kTW;
-    const int tx0 = edges ? G.nBandTx : 0;
-    const int k = item - (edges ? G.edgeBase : G.stripBase);
-    const int tx = tx0 + k % (tilesX - tx0), tyg = k / (tilesX - tx0);
+    const int k = item - (rest ? G.restBase : G.stripBase);
+    const int tx = k % tilesX, tyg = k / tilesX;
     if (stripIsInterior(a, tx)) stencilStripImpl<T, H, V, RPW, Xform::Identity, true>(a, w, tile, tx, tyg);
     else stencilStripImpl<T, H, V, RPW, Xform::Identity, false>(a, w, tile, tx, tyg);
 }
 
-// Band walker over the interior strips [0, nBandTx) of every grid.
+// Band walker over the grids it applies to.
 template <typename T, int H, int V, int RPW>
 __global__ __launch_bounds__(kLanes) void batchBandKernel(const BatchDev* __restrict__ grids,
                                                           const int* __restrict__ itemGrid,
@@ -130,10 +129,7 @@ __global__ __launch_bounds__(kLanes) void batchBandKernel(const BatchDev* __rest
     const BatchDev& G = grids[itemGrid[item]];
     StencilLaunch a = gridLaunch(G, parity, sizeof(T) == 8 ? Dtype::F64 : Dtype::F32, weights, H,
                                  L, V, Tt, RPW, chunks);
-    a.nStripTx = G.nBandTx;
-    Lds<T>* r = (Lds<T>*)ring;
-    if (G.ny % RPW == 0) bandWalk<T, H, V, RPW, true>(a, w, r, item - G.bandBase);
-    else bandWalk<T, H, V, RPW, false>(a, w, r, item - G.bandBase);
+    bandWalk<T, H, V, RPW>(a, w, (Lds<T>*)ring, item - G.bandBase);
 }
 
 }  // namespace dev
@@ -151,9 +147,9 @@ struct custenBatch {
     std::vector<BatchDev> host;
     std::vector<int> strips;  // strips per grid
     int totalStrips = 0;
-    int totalBand = 0, totalEdge = 0;  // band items and edge-strip items (band mode)
+    int totalBand = 0, totalRest = 0;  // band items and the unwalked grids' strips (band mode)
     BatchDev* dGrids = nullptr;
-    // owning grid of every item: all strips, band items, edge-strip items
+    // owning grid of every item: all strips, the unwalked grids' strips, band items
     int* dItemGrid[3] = {nullptr, nullptr, nullptr};
     size_t itemCap[3] = {0, 0, 0};
     double* dWeights = nullptr;
@@ -189,7 +185,7 @@ hipError_t launchOne(const custenBatch* b, const BatchDev* grids, int firstItem,
 }
 
 // kind 0: strip kernel over items [firstItem, +nItems) of the all-strips
-// table; 1: strip kernel over the edge-strip table; 2: band walker over the
+// table; 1: strip kernel over the unwalked grids' strips; 2: band walker over the
 // band table (firstItem must be 0 for kinds 1 and 2).
 hipError_t launchItems(const custenBatch* b, int firstItem, int nItems, int parity, hipStream_t st,
                        int kind = 0)
@@ -216,46 +212,52 @@ hipError_t launchItems(const custenBatch* b, int firstItem, int nItems, int pari
 
 // Item tables for a tile configuration (host copy and device copy): all
 // strips (per-grid loop and strip-only fused steps) and, with the band
-// walker, its band items and the remaining edge strips.  A grid's strips are
-// walked by bands when its rows are pair-aligned and its height allows one
-// wrap correction per row (ny >= V + rows per wave).
+// walker, the band items of the grids it applies to (at least a strip wide
+// and a chunk and the stencil high) and the strips of the others.
 hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
 {
     b->rpw = rpw;
     b->chunks = chunks;
     b->band = band;
-    int64_t strips = 0, bands = 0, edges = 0;
-    for (int g = 0; g < b->numGrids; g++) {
-        BatchDev& d = b->host[g];
+    int64_t strips = 0, bands = 0, rest = 0;
+    for (int gi = 0; gi < b->numGrids; gi++) {
+        BatchDev& d = b->host[gi];
         d.stripBase = (int)strips;
-        b->strips[g] = stripsFor(d.nx, d.ny, rpw, chunks);
-        strips += b->strips[g];
-        const int tilesX = (d.nx + dev::kTW - 1) / dev::kTW;
-        d.nBandTx = (band && d.vec && d.ny >= b->V + rpw) ? d.nx / dev::kTW : 0;
+        b->strips[gi] = stripsFor(d.nx, d.ny, rpw, chunks);
+        strips += b->strips[gi];
+        StencilLaunch one{};
+        one.ny = one.wy1 = one.rows.rowWrap = d.ny;
+        one.wx1 = d.nx;
+        one.V = b->V;
+        one.rows.wrap = 1;
+        one.chunks = chunks;
+        d.walked = band && dev::bandApplies(one, rpw) ? 1 : 0;
         d.bandBase = (int)bands;
-        d.edgeBase = (int)edges;
-        const int bandRows = rpw * chunks;
-        const int groupRows = dev::kWaves * rpw * chunks;
-        bands += (int64_t)d.nBandTx * ((d.ny + bandRows - 1) / bandRows);
-        edges += (int64_t)(tilesX - d.nBandTx) * ((d.ny + groupRows - 1) / groupRows);
+        d.restBase = (int)rest;
+        if (d.walked) {
+            const dev::BandGrid g = dev::bandGrid(one, rpw);
+            bands += (int64_t)g.strips * g.bands;
+        } else {
+            rest += b->strips[gi];
+        }
     }
     if (strips > (int64_t)0x7fffffff || bands > (int64_t)0x7fffffff ||
-        edges > (int64_t)0x7fffffff)
+        rest > (int64_t)0x7fffffff)
         return hipErrorInvalidValue;
     b->totalStrips = (int)strips;
     b->totalBand = (int)bands;
-    b->totalEdge = (int)edges;
+    b->totalRest = (int)rest;
     // owning grid of every item of the three tables
     std::vector<int> owner[3];
     owner[0].reserve(b->totalStrips);
-    owner[1].reserve(b->totalEdge);
+    owner[1].reserve(b->totalRest);
     owner[2].reserve(b->totalBand);
     for (int g = 0; g < b->numGrids; g++) {
         const BatchDev& d = b->host[g];
         const int nBand = (g + 1 < b->numGrids ? b->host[g + 1].bandBase : b->totalBand) - d.bandBase;
-        const int nEdge = (g + 1 < b->numGrids ? b->host[g + 1].edgeBase : b->totalEdge) - d.edgeBase;
+        const int nRest = (g + 1 < b->numGrids ? b->host[g + 1].restBase : b->totalRest) - d.restBase;
         owner[0].insert(owner[0].end(), b->strips[g], g);
-        owner[1].insert(owner[1].end(), nEdge, g);
+        owner[1].insert(owner[1].end(), nRest, g);
         owner[2].insert(owner[2].end(), nBand, g);
     }
     for (int k = 0; k < 3; k++) {
@@ -279,12 +281,12 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
 }
 
 // One fused step at parity p: one launch over all strips, or the band walker
-// then the edge strips.
+// then the strips of the grids that are not walked.
 hipError_t enqueueStep(const custenBatch* b, int p, hipStream_t st)
 {
     if (!b->band) return launchItems(b, 0, b->totalStrips, p, st, 0);
     hipError_t e = launchItems(b, 0, b->totalBand, p, st, 2);
-    if (e == hipSuccess) e = launchItems(b, 0, b->totalEdge, p, st, 1);
+    if (e == hipSuccess) e = launchItems(b, 0, b->totalRest, p, st, 1);
     return e;
 }
 

@@ -59,8 +59,8 @@ struct StencilLaunch {
     int stripTx0, nStripTx;
     int edgeList;
     int edgeTx[4];
-    // 1: interior strips run the band walker (identity transform): one wave
-    // per rowsPerWave * chunks rows of a strip
+    // 1: the band walker where it applies: one wave per rowsPerWave * chunks
+    // rows of a 128-column strip of the written window
     int band;
 };
 

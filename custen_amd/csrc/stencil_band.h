@@ -13,9 +13,18 @@
 // chunks are never copied.  Completion is tracked with the vector-memory
 // counter, which retires loads and stores in issue order: before chunk c the
 // wave waits until no more than (loads issued after chunk c's) + (stores
-// issued after chunk c's) operations are outstanding.  A chunk whose stores
-// did not take the one-store-per-row path (write-masked or ragged rows)
-// makes the following waits drain the counter instead.
+// issued after chunk c's) operations are outstanding.
+//
+// Every point of a walked strip is written, so there are no store masks: the
+// walked strips tile the written columns of the launch, the last one ending
+// at the last written column (it overlaps its neighbour when their number is
+// not a multiple of 128), and the chunks tile the written rows, the last band
+// ending at the last of them.  Points in an overlap are computed by both
+// waves from the same values in the same order.  A strip may start at any
+// column and rows at any alignment of an element: the loads and stores need
+// element alignment only.  At 4099 x 3001 (5x5, FP64, written window inside a
+// one-cell border on odd rows) the apply takes 32.0 us (197 MB, 6.1
+// TB/s), against 49.4 when such rows took the strip kernel's per-element path.
 //
 // Arithmetic is the fma chain of the other stencil kernels (row j outer,
 // column i inner, from 0.0), so every configuration gives identical bits.
@@ -84,17 +93,22 @@ __device__ __forceinline__ void ldsDma4(const Glob<unsigned>* g, Lds<T>* l)
 
 // FP64 stencils of more than 36 points have more weights than the scalar
 // registers hold next to the walker's own state; held for the whole walk they
-// are spilled and read back lane by lane.  The unmasked (FULL) walk of those
-// stencils instead loads each weight row from the scalar cache just before
-// its FMAs (the weights are not written during a launch, so the constant
-// address space applies).  The masked walk keeps resident weights: with its
-// store masks in the loop the compiler spilled more when streaming.
-template <typename T, int H, int V, bool FULL>
-constexpr bool kStreamWeights = FULL && sizeof(T) == 8 && H * V > 36;
+// are spilled and read back lane by lane.  The walk of those stencils instead
+// loads each weight row from the scalar cache just before its FMAs (the
+// weights are not written during a launch, so the constant address space
+// applies).
+template <typename T, int H, int V>
+constexpr bool kStreamWeights = sizeof(T) == 8 && H * V > 36;
 
 // FP32 stencils of more than 36 points: the weights (converted from the
 // FP64 array on the vector unit) stay in vector registers, 49 or 81 of them,
 // instead of being moved to scalar registers that then spill.
+// A pair of elements at element alignment.
+template <typename T> struct ElemPair;
+template <> struct ElemPair<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct ElemPair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <typename T> using ElemVec2 = typename ElemPair<T>::type;
+
 template <typename T, int H, int V>
 constexpr bool kWeightsInVgprs = sizeof(T) == 4 && H * V > 36;
 
@@ -129,17 +143,41 @@ struct BandShape {
     static constexpr int LDS_BYTES = S * LD * (int)sizeof(T);
 };
 
-// Band walk of wave g of a launch (one wave per workgroup): interior strip
-// stripTx0 + g % nStripTx (or, with edgeList, edgeTx[g % nStripTx]) over
-// region rows [band * RPW * chunks, ...) with band = g / nStripTx.  `ring` is the wave's BandShape::S x LD LDS ring and
-// `w` the H*V weights; X the point-wise transform of the values read.
-// Requirements (checked by the host): the strip is interior (full 128
-// columns, pair-aligned rows), and wrapped row indices need at most one
-// correction for every row the band touches.  FULL (also decided by the
-// host): every point of every walked strip is written and the region height
-// is a multiple of RPW, so each chunk stores RPW whole rows.  With
-// kStreamWeights the weights come from a.weights and `w` is not read.
-template <typename T, int H, int V, int RPW, bool FULL, Xform X = Xform::Identity>
+// What a launch of the band walker covers: written columns [xa, xb) in strips
+// of 128 and written rows [ya, yb) in chunks of rpw rows, `chunks` to a band.
+struct BandGrid {
+    int xa, xb, ya, yb, strips, total, chunks, bands;
+};
+__host__ __device__ inline BandGrid bandGrid(const StencilLaunch& a, int rpw)
+{
+    BandGrid g;
+    g.xa = a.wx0;
+    g.xb = a.wx1;
+    g.ya = a.wy0 > a.yGlobal0 ? a.wy0 - a.yGlobal0 : 0;
+    g.yb = a.wy1 - a.yGlobal0 < a.ny ? a.wy1 - a.yGlobal0 : a.ny;
+    const int rows = g.yb - g.ya;
+    g.strips = (g.xb - g.xa + kTW - 1) / kTW;
+    g.total = (rows + rpw - 1) / rpw;
+    // fewer rows than a band: the ragged last chunk gets a band of its own,
+    // which ends at the last row without starting before the first
+    g.chunks = a.chunks < rows / rpw ? a.chunks : rows / rpw;
+    g.bands = g.chunks > 0 ? (g.total + g.chunks - 1) / g.chunks : 0;
+    return g;
+}
+// The walker's conditions: a full strip of written columns, a full chunk of
+// written rows, and at most one wrap correction for every row it touches.
+__host__ __device__ inline bool bandApplies(const StencilLaunch& a, int rpw)
+{
+    const BandGrid g = bandGrid(a, rpw);
+    return g.xb - g.xa >= kTW && g.yb - g.ya >= rpw &&
+           (!a.rows.wrap || (a.rows.rowWrap >= a.V + rpw && a.ny <= a.rows.rowWrap));
+}
+
+// Band walk of wave g of a launch (one wave per workgroup): strip
+// g % strips, band g / strips.  `ring` is the wave's BandShape::S x LD LDS ring
+// and `w` the H*V weights; X the point-wise transform of the values read.
+// With kStreamWeights the weights come from a.weights and `w` is not read.
+template <typename T, int H, int V, int RPW, Xform X = Xform::Identity>
 __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H * V],
                                          Lds<T>* __restrict__ ring, int g)
 {
@@ -148,21 +186,20 @@ __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H 
     constexpr int HL = BS::HALO_LANES;
 
     const int lane = threadIdx.x;
-    const int tx = a.edgeList ? a.edgeTx[g % a.nStripTx] : a.stripTx0 + g % a.nStripTx;
-    const int band = g / a.nStripTx;
-    const int bandRows = RPW * a.chunks;
-    const int yS = band * bandRows;
-    if (yS >= a.ny) return;
-    const int yE = min(yS + bandRows, a.ny);
-    const int nChunks = (yE - yS + RPW - 1) / RPW;
+    const BandGrid bg = bandGrid(a, RPW);
+    const int strip = g % bg.strips, band = g / bg.strips;
+    const int nChunks = min(bg.chunks, bg.total - band * bg.chunks);
+    const int yS = min(bg.ya + band * bg.chunks * RPW, bg.yb - nChunks * RPW);
 
     const Glob<T>* __restrict__ in = globalPtr<T>(a.in);
     Glob<T>* __restrict__ out = globalPtr<T>(a.out);
     const int nx = a.nx;
-    const int x0 = tx * kTW;
+    const int x0 = min(bg.xa + strip * kTW, bg.xb - kTW);
     const int L = a.L;
     const int R = H - 1 - L;
-    const bool fullRow = x0 >= a.wx0 && x0 + kTW <= a.wx1;
+    // x-np (V == 1): the last strip's waves also write 0 to the R columns right
+    // of it
+    const bool zeros = V == 1 && a.zeroRight && strip == bg.strips - 1;
 
     // halo columns staged for this lane (lanes < HL, one dword each)
     const int hcol = sizeof(T) == 8 ? lane >> 1 : lane;
@@ -225,10 +262,9 @@ __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H 
     }
 
     int slotBase = 0;
-    unsigned inexact = 0;  // bit i: chunk c-1-i did not store one row per instruction
     for (int c = 0; c < nChunks; c++) {
-        if (!FULL && (inexact & ((1u << D) - 1u))) {
-            waitVmcnt<0>();
+        if (zeros) {
+            waitVmcnt<0>();  // its extra stores are not in the count
         } else {
             const int la = min(c + D - 1, nChunks - 1) - c;
             const int sa = min(c, D);
@@ -270,7 +306,7 @@ __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H 
                 const int j = ir - r;
                 if (j >= 0 && j < V) {
                     T wr[H];
-                    if constexpr (kStreamWeights<T, H, V, FULL>) {
+                    if constexpr (kStreamWeights<T, H, V>) {
                         loadWeightRow<H>(a.weights, j, wr, acc[r][1]);
                     } else {
 #pragma unroll
@@ -285,29 +321,13 @@ __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H 
             }
         }
 
-        if constexpr (FULL) {
 #pragma unroll
-            for (int r = 0; r < RPW; r++) {
-                using V2 = typename Vec2<T>::type;
-                const V2 o = {acc[r][0], acc[r][1]};
-                __builtin_nontemporal_store(
-                    o, reinterpret_cast<Glob<V2>*>(out + (int64_t)(yS + c * RPW + r) * a.ldOut +
-                                                   x0 + 2 * lane));
-            }
-        } else {
-            bool exact = fullRow;
-#pragma unroll
-            for (int r = 0; r < RPW; r++) {
-                const int gy = yS + c * RPW + r;
-                const int gyg = a.yGlobal0 + gy;
-                if (gy >= yE || gyg < a.wy0 || gyg >= a.wy1) {
-                    exact = false;
-                    continue;
-                }
-                storeLane<T, 2>(out + (int64_t)gy * a.ldOut, x0 + 2 * lane, acc[r], fullRow, nx,
-                                a.wx0, a.wx1, a.zeroRight, R);
-            }
-            inexact = (inexact << 1) | (exact ? 0u : 1u);
+        for (int r = 0; r < RPW; r++) {
+            const typename Vec2<T>::type v = {acc[r][0], acc[r][1]};
+            Glob<T>* orow = out + (int64_t)(yS + c * RPW + r) * a.ldOut;
+            __builtin_nontemporal_store(ElemVec2<T>(v),
+                                        reinterpret_cast<Glob<ElemVec2<T>>*>(orow + x0 + 2 * lane));
+            if (zeros && lane < R) orow[nx - R + lane] = T(0);
         }
         slotBase += RPW;
         if (slotBase >= S) slotBase -= S;
@@ -315,13 +335,13 @@ __device__ __forceinline__ void bandWalk(const StencilLaunch& a, const T (&w)[H 
 }
 
 // Single-region launch: one wave per workgroup, waves in XCD-aware order.
-template <typename T, int H, int V, int RPW, bool FULL, Xform X = Xform::Identity>
+template <typename T, int H, int V, int RPW, Xform X = Xform::Identity>
 __global__ __launch_bounds__(kLanes) void stencilBand(StencilLaunch a)
 {
     using BS = BandShape<T, H, V, RPW>;
     __shared__ __attribute__((aligned(16))) T ring[BS::S * BS::LD];
     T w[H * V];
-    if constexpr (!kStreamWeights<T, H, V, FULL>) {
+    if constexpr (!kStreamWeights<T, H, V>) {
 #pragma unroll
         for (int k = 0; k < H * V; k++) w[k] = static_cast<T>(a.weights[k]);
     }
@@ -335,7 +355,7 @@ __global__ __launch_bounds__(kLanes) void stencilBand(StencilLaunch a)
             w[k] = o;
         }
     }
-    bandWalk<T, H, V, RPW, FULL, X>(a, w, (Lds<T>*)ring, xcdRemap(blockIdx.x, gridDim.x));
+    bandWalk<T, H, V, RPW, X>(a, w, (Lds<T>*)ring, xcdRemap(blockIdx.x, gridDim.x));
 }
 
 }  // namespace dev

@@ -386,6 +386,8 @@ namespace {
 
 constexpr int kDefaultRPW = 8;
 constexpr int kDefaultChunks = 4;
+// From this many points on, bands of 8 rows still make 8 waves per CU.
+constexpr int64_t kLongBandPoints = int64_t(1) << 21;
 
 template <typename T>
 bool pairAligned(const void* p, int64_t ld)
@@ -401,14 +403,30 @@ int gridSize(int nx, int ny, int TH, int chunks)
     return tilesX * tilesY;
 }
 
-// Interior column strips run the FAST kernel (or the band walker), the edge
-// strips the general one: by list when there are at most four, otherwise (no
+// The band walker takes the whole written window when it is asked for and
+// applies.  Otherwise interior column strips run the FAST kernel, the edge
+// strips the general one: by list when there are at most four, else (no
 // interior strip at all: unaligned rows, or a periodic grid lower than the
 // stencil) as the contiguous ranges left and right of the interior.
 template <typename T, int H, int V, int RPW, Xform X, int CPL = 2>
 hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
 {
     StencilLaunch s = in;
+    // band walker: every weight stencil shape, and the cube-minus point
+    // function on its xy shapes 3x3 and 5x5
+    constexpr bool bandShape =
+        X == Xform::Identity ||
+        (X == Xform::CubeMinus && H == V && (H == 3 || H == 5) && sizeof(T) == 8);
+    if constexpr (bandShape && CPL == 2 && (RPW == 4 || RPW == 8)) {
+        if (s.band && dev::bandApplies(s, RPW)) {
+            const dev::BandGrid g = dev::bandGrid(s, RPW);
+            const int64_t waves = (int64_t)g.strips * g.bands;
+            if (waves > 0x7fffffff) return hipErrorInvalidValue;
+            hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, X>), dim3((unsigned)waves),
+                               dim3(dev::kLanes), 0, st, s);
+            return hipGetLastError();
+        }
+    }
     const int tw = dev::kLanes * CPL;
     const int tilesX = (s.nx + tw - 1) / tw;
     const int rowsPerGroup = dev::kWaves * RPW * s.chunks;
@@ -455,94 +473,6 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
         s.edgeList = 0;
         s.stripTx0 = lo;
         s.nStripTx = hi - lo;
-        // band walker: every weight stencil shape, and the cube-minus point
-        // function on its xy shapes 3x3 and 5x5
-        constexpr bool bandShape =
-            X == Xform::Identity ||
-            (X == Xform::CubeMinus && H == V && (H == 3 || H == 5) && sizeof(T) == 8);
-        if constexpr (bandShape && CPL == 2 && (RPW == 4 || RPW == 8)) {
-            // band walker: every row it touches must need at most one wrap
-            if (s.band && (!s.rows.wrap || (s.rows.rowWrap >= s.V + RPW && s.ny <= s.rows.rowWrap))) {
-                const int bandRows = RPW * s.chunks;
-                const int64_t waves = (int64_t)s.nStripTx * ((s.ny + bandRows - 1) / bandRows);
-                if (waves > 0x7fffffff) return hipErrorInvalidValue;
-                // every walked point written, whole chunks: no store masks
-                const bool full = lo * dev::kTW >= s.wx0 && hi * dev::kTW <= s.wx1 &&
-                                  s.yGlobal0 >= s.wy0 && s.yGlobal0 + s.ny <= s.wy1 &&
-                                  s.ny % RPW == 0;
-                if (full || !dev::kStreamWeights<T, H, V, true>) {
-                    if (full)
-                        hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, true, X>),
-                                           dim3((unsigned)waves), dim3(dev::kLanes), 0, st, s);
-                    else
-                        hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, false, X>),
-                                           dim3((unsigned)waves), dim3(dev::kLanes), 0, st, s);
-                    return hipGetLastError();
-                }
-                // Stencils whose masked walk keeps resident (spilled) weights:
-                // the unmasked walk serves the strips whose every column is
-                // written, [xa, xb), over the whole chunks of the written rows
-                // [ya, ya + yFull); the masked walk serves the ragged rows and
-                // the strips at the column window's edges.  Rows outside the
-                // row window are not written and are skipped.  A row offset
-                // needs clamped rows (wrapped rows are addressed from region
-                // row 0).
-                int xa = lo, xb = hi;
-                while (xa < xb && xa * dev::kTW < s.wx0) xa++;
-                while (xb > xa && xb * dev::kTW > s.wx1) xb--;
-                const int ya = std::max(0, s.wy0 - s.yGlobal0);
-                const int yb = std::min(s.ny, s.wy1 - s.yGlobal0);
-                int yFull = yb > ya ? (yb - ya) / RPW * RPW : 0;
-                if (s.rows.wrap && (ya != 0 || yFull != s.ny)) yFull = 0;
-                auto walk = [&](bool fullWalk, const StencilLaunch& strips, int y0,
-                                int n) -> hipError_t {
-                    if (strips.nStripTx <= 0 || n <= 0) return hipSuccess;
-                    StencilLaunch t = strips;
-                    t.ny = n;
-                    if (y0 > 0) {
-                        t.in = static_cast<const char*>(s.in) + (int64_t)y0 * s.ldIn * sizeof(T);
-                        t.out = static_cast<char*>(s.out) + (int64_t)y0 * s.ldOut * sizeof(T);
-                        t.yGlobal0 = s.yGlobal0 + y0;
-                        t.rows.rowMin = s.rows.rowMin - y0;
-                        t.rows.rowMax = s.rows.rowMax - y0;
-                    }
-                    const unsigned w =
-                        (unsigned)((int64_t)t.nStripTx * ((n + bandRows - 1) / bandRows));
-                    if (fullWalk)
-                        hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, true, X>), dim3(w),
-                                           dim3(dev::kLanes), 0, st, t);
-                    else
-                        hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, false, X>), dim3(w),
-                                           dim3(dev::kLanes), 0, st, t);
-                    return hipGetLastError();
-                };
-                auto range = [&](int tx0, int ntx) {
-                    StencilLaunch t = s;
-                    t.edgeList = 0;
-                    t.stripTx0 = tx0;
-                    t.nStripTx = ntx;
-                    return t;
-                };
-                if (yFull == 0 || xb <= xa) return walk(false, range(lo, hi - lo), 0, s.ny);
-                hipError_t err;
-                if ((err = walk(true, range(xa, xb - xa), ya, yFull)) != hipSuccess) return err;
-                if ((err = walk(false, range(xa, xb - xa), ya + yFull, yb - ya - yFull)) !=
-                    hipSuccess)
-                    return err;
-                const int nSide = (xa - lo) + (hi - xb);
-                if (nSide <= 4) {
-                    // both edges in one launch
-                    StencilLaunch e = s;
-                    e.edgeList = 1;
-                    e.nStripTx = 0;
-                    for (int tx = lo; tx < hi; tx++)
-                        if (tx < xa || tx >= xb) e.edgeTx[e.nStripTx++] = tx;
-                    return walk(false, e, ya, yb - ya);
-                }
-                if ((err = walk(false, range(lo, xa - lo), ya, yb - ya)) != hipSuccess) return err;
-                return walk(false, range(xb, hi - xb), ya, yb - ya);
-            }
-        }
         hipLaunchKernelGGL((dev::stencilFixed<T, H, V, RPW, X, true, CPL>),
                            dim3(s.nStripTx * tilesY), dim3(dev::kThreads), 0, st, s);
         return hipGetLastError();
@@ -626,6 +556,14 @@ hipError_t launchStencil(const StencilLaunch& in, hipStream_t st)
     StencilLaunch s = in;
     if (s.nx <= 0 || s.ny <= 0) return hipSuccess;
     if (s.H < 1 || s.V < 1 || s.H > 65 || s.V > 65) return hipErrorInvalidValue;
+    // No configuration given (grids below the autotuner's size, streamed
+    // tiles, capture before the first Compute): the band walker, with bands
+    // short enough to put a few waves on every CU.
+    if (s.rowsPerWave == 0 && s.chunks == 0 && s.colsPerLane == 0 && !s.band) {
+        s.band = 1;
+        s.rowsPerWave = 4;
+        s.chunks = (int64_t)s.nx * s.ny >= kLongBandPoints ? 2 : 1;
+    }
     if (s.colsPerLane != 1) s.colsPerLane = 2;
     if (s.colsPerLane == 1) {
         if (s.rowsPerWave != 8 && s.rowsPerWave != 16) s.rowsPerWave = 16;
@@ -651,7 +589,6 @@ hipError_t launchFun(const FunLaunch& in, hipStream_t st)
     if (f.nx <= 0 || f.ny <= 0) return hipSuccess;
     if (f.H < 1 || f.V < 1 || f.H > 65 || f.V > 65) return hipErrorInvalidValue;
     if (f.numCoe < 0 || f.numCoe > dev::kMaxCoe) return hipErrorInvalidValue;
-    if (f.chunks <= 0) f.chunks = kDefaultChunks;
     f.vecIn = pairAligned<double>(f.in, f.ldIn);
 
     // Built-in xy functions are weighted sums (of u or of u^3 - u): run them on
@@ -686,6 +623,7 @@ hipError_t launchFun(const FunLaunch& in, hipStream_t st)
         s.band = f.band;
         return launchStencil(s, st);
     }
+    if (f.chunks <= 0) f.chunks = kDefaultChunks;
 
     const int TH = dev::kWaves * dev::kFunRPW;
     const int grid = gridSize(f.nx, f.ny, TH, f.chunks);

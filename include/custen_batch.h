@@ -31,8 +31,8 @@ int custenBatchRun(custenBatch* batch, int steps, int mode, hipStream_t stream);
 int custenBatchParity(const custenBatch* batch);
 /* Tile configuration of the fused steps (results do not depend on it):
  * band = 0: strip kernel, rowsPerWave 4 or 8 and chunks >= 1 row chunks per
- * workgroup; band = 1: band walker for the interior 128-column strips of
- * every grid (chunks per band), strip kernel for the rest.  Replaces the
+ * workgroup; band = 1: band walker (chunks per band) for every grid at least
+ * 128 columns wide and a chunk high, strip kernel for the rest.  Replaces the
  * autotuner's choice; graphs captured before are discarded.  Waits for the
  * batch's earlier work on its own stream. */
 int custenBatchSetTileConfig(custenBatch* batch, int rowsPerWave, int chunks, int band);
