@@ -1,8 +1,9 @@
 // batch.hip -- many independent periodic xy grids of uneven sizes advanced
-// together: one launch per step covers every strip of every grid (the
-// workgroup finds its grid by binary search over the strip prefix sums), and
-// a whole multi-step run is captured once into a HIP graph and replayed.
-// With the band walker selected, a step walks every grid that is at least a
+// together: one launch covers every strip of every grid (an item table gives
+// each workgroup its grid), three steps to a launch (stencil_steps.h) and the
+// last one to three of a run one each, and a whole multi-step run is captured
+// once into a HIP graph and replayed.
+// With the band walker selected, a single step walks every grid that is at least a
 // strip wide and a chunk high (one wave per band, found the same way); a
 // second launch runs the strip kernel over the smaller grids, if any.  The
 // per-grid launch loop (one launch per grid per step) is kept as the baseline
@@ -22,6 +23,7 @@
 #include "plan_internal.h"
 #include "stencil_band.h"
 #include "stencil_body.h"
+#include "stencil_steps.h"
 #include "tuner.h"
 
 #pragma clang fp contract(off)
@@ -40,6 +42,10 @@ struct BatchDev {
     int walked;
     int bandBase;   // first band item (wave) of this grid
     int restBase;   // first strip item of this grid, if it is not walked
+    // passes of several steps: the same for the grids stepsWalk applies to
+    int stepped;
+    int stepsBase;
+    int stepsRestBase;
 };
 
 namespace dev {
@@ -86,8 +92,8 @@ __device__ __forceinline__ StencilLaunch gridLaunch(const BatchDev& G, int parit
     return a;
 }
 
-// Strip kernel over every strip of every grid (rest = 0) or over those of the
-// grids that are not walked (rest = 1).
+// Strip kernel over every strip of every grid (rest = 0), of the grids that
+// are not walked (1) or of those that passes of several steps leave out (2).
 // itemGrid[item] is the grid that owns the item (built on the host with the
 // item tables, so a workgroup finds its grid with one load).
 template <typename T, int H, int V, int RPW>
@@ -106,7 +112,7 @@ __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restri
     const StencilLaunch a = gridLaunch(G, parity, sizeof(T) == 8 ? Dtype::F64 : Dtype::F32,
                                        weights, H, L, V, Tt, RPW, chunks);
     const int tilesX = (G.nx + kTW - 1) / kTW;
-    const int k = item - (rest ? G.restBase : G.stripBase);
+    const int k = item - (rest == 0 ? G.stripBase : rest == 1 ? G.restBase : G.stepsRestBase);
     const int tx = k % tilesX, tyg = k / tilesX;
     if (stripIsInterior(a, tx)) stencilStripImpl<T, H, V, RPW, Xform::Identity, true>(a, w, tile, tx, tyg);
     else stencilStripImpl<T, H, V, RPW, Xform::Identity, false>(a, w, tile, tx, tyg);
@@ -132,10 +138,40 @@ __global__ __launch_bounds__(kLanes) void batchBandKernel(const BatchDev* __rest
     bandWalk<T, H, V, RPW>(a, w, (Lds<T>*)ring, item - G.bandBase);
 }
 
+// kFusedSteps steps of the grids stepsWalk applies to.
+template <typename T, int H, int V>
+__global__ __launch_bounds__(kLanes) void batchStepsKernel(const BatchDev* __restrict__ grids,
+                                                           const int* __restrict__ itemGrid,
+                                                           int parity,
+                                                           const double* __restrict__ weights,
+                                                           int L, int Tt, int most)
+{
+    __shared__ __attribute__((aligned(16))) T lds[StepsShape<T, H, V, kFusedSteps>::ELEMS];
+    T w[H * V];
+#pragma unroll
+    for (int k = 0; k < H * V; k++) w[k] = static_cast<T>(weights[k]);
+    const int item = xcdRemap(blockIdx.x, gridDim.x);
+    const BatchDev& G = grids[itemGrid[item]];
+    const void* in = parity ? G.out : G.in;
+    void* out = parity ? const_cast<void*>(G.in) : G.out;
+    stepsWalk<T, H, V, kFusedSteps>(globalPtr<T>(in), globalPtr<T>(out), G.nx, G.ny, L, Tt, w,
+                                    (Lds<T>*)lds, most, item - G.stepsBase);
+}
+
 }  // namespace dev
 }  // namespace custen
 
 using namespace custen;
+
+// Item tables of a batch (owning grid of every item).
+enum ItemKind {
+    kAllStrips = 0,   // every strip
+    kRestStrips = 1,  // strips of the grids the band walker leaves out
+    kBands = 2,       // the band walker's waves
+    kSteps = 3,       // waves of a pass of several steps
+    kStepsRest = 4,   // strips of the grids such a pass leaves out
+    kItemKinds = 5
+};
 
 struct custenBatch {
     int device = 0;
@@ -146,12 +182,11 @@ struct custenBatch {
     bool band = false;        // fused steps use the band walker for interior strips
     std::vector<BatchDev> host;
     std::vector<int> strips;  // strips per grid
-    int totalStrips = 0;
-    int totalBand = 0, totalRest = 0;  // band items and the unwalked grids' strips (band mode)
+    int total[kItemKinds] = {};
+    int stepRows = 16;        // most rows per band of a pass of several steps
     BatchDev* dGrids = nullptr;
-    // owning grid of every item: all strips, the unwalked grids' strips, band items
-    int* dItemGrid[3] = {nullptr, nullptr, nullptr};
-    size_t itemCap[3] = {0, 0, 0};
+    int* dItemGrid[kItemKinds] = {};
+    size_t itemCap[kItemKinds] = {};
     double* dWeights = nullptr;
     int parity = 0;           // 1: the current input is the original output side
     bool tuned = false;
@@ -170,31 +205,31 @@ int stripsFor(int nx, int ny, int rpw, int chunks)
 }
 
 template <typename T, int H, int V, int RPW>
-hipError_t launchOne(const custenBatch* b, const BatchDev* grids, int firstItem, int nItems,
-                     int parity, int kind, hipStream_t st)
+hipError_t launchOne(const custenBatch* b, int firstItem, int nItems, int parity, ItemKind kind,
+                     hipStream_t st)
 {
-    if (kind == 2)
+    const int* owner = b->dItemGrid[kind];
+    if (kind == kBands)
         hipLaunchKernelGGL((dev::batchBandKernel<T, H, V, RPW>), dim3(nItems), dim3(dev::kLanes),
-                           0, st, grids, b->dItemGrid[2], parity, b->dWeights, b->L, b->T,
-                           b->chunks);
+                           0, st, b->dGrids, owner, parity, b->dWeights, b->L, b->T, b->chunks);
+    else if (kind == kSteps)
+        hipLaunchKernelGGL((dev::batchStepsKernel<T, H, V>), dim3(nItems), dim3(dev::kLanes), 0, st,
+                           b->dGrids, owner, parity, b->dWeights, b->L, b->T, b->stepRows);
     else
         hipLaunchKernelGGL((dev::batchKernel<T, H, V, RPW>), dim3(nItems), dim3(dev::kThreads), 0,
-                           st, grids, b->dItemGrid[kind], firstItem, parity, b->dWeights, b->L,
-                           b->T, b->chunks, kind);
+                           st, b->dGrids, owner, firstItem, parity, b->dWeights, b->L, b->T,
+                           b->chunks, kind == kAllStrips ? 0 : kind == kRestStrips ? 1 : 2);
     return hipGetLastError();
 }
 
-// kind 0: strip kernel over items [firstItem, +nItems) of the all-strips
-// table; 1: strip kernel over the unwalked grids' strips; 2: band walker over the
-// band table (firstItem must be 0 for kinds 1 and 2).
+// Items [firstItem, +nItems) of a table (firstItem is 0 for all but kAllStrips).
 hipError_t launchItems(const custenBatch* b, int firstItem, int nItems, int parity, hipStream_t st,
-                       int kind = 0)
+                       ItemKind kind = kAllStrips)
 {
     if (nItems <= 0) return hipSuccess;
-    const BatchDev* g = b->dGrids;
-#define CUSTEN_BATCH_CASE(TT, HH, VV, RR)                                              \
-    if (b->H == HH && b->V == VV && b->rpw == RR)                                      \
-        return launchOne<TT, HH, VV, RR>(b, g, firstItem, nItems, parity, kind, st);
+#define CUSTEN_BATCH_CASE(TT, HH, VV, RR)         \
+    if (b->H == HH && b->V == VV && b->rpw == RR) \
+        return launchOne<TT, HH, VV, RR>(b, firstItem, nItems, parity, kind, st);
     if (b->dtype == Dtype::F64) {
         CUSTEN_BATCH_CASE(double, 5, 5, 8)
         CUSTEN_BATCH_CASE(double, 5, 5, 4)
@@ -210,21 +245,76 @@ hipError_t launchItems(const custenBatch* b, int firstItem, int nItems, int pari
     return hipErrorInvalidValue;
 }
 
+hipError_t launchAll(const custenBatch* b, ItemKind kind, int parity, hipStream_t st)
+{
+    return launchItems(b, 0, b->total[kind], parity, st, kind);
+}
+
+// Several steps in one pass pay once the two sides no longer stay in the L2s
+// (8 x 4 MiB): single steps then wait for memory, and a pass takes a third of
+// its traffic.  In L2 a single step costs 4-6 us and a pass is bound by its
+// chain of rows.  31 steps, single against passes, in us, by MiB a side:
+//   FP64 5x5   16: 196, 288   32:  470, 412   64:  957, 699   128: 1720, 1164
+//   FP32 5x5   16: 220, 280   32:  560, 429   64: 1056, 707
+//   FP64 3x3   16: 174, 160   32:  495, 238   64:  918, 434   128: 1668, 760
+//   FP32 3x3   16: 188, 165   32:  516, 279   64:  979, 552
+constexpr int64_t kStepBytes5 = 24 << 20, kStepBytes3 = 16 << 20;
+// Most rows of a pass's band.  Short bands repeat more rows (V - 1 for each
+// step) and long ones come in few rounds of waves.  In FP64 a batch takes the
+// length of 128, 64, 32, 16 for which rounds times rows is least, where a wave
+// holds 11 KB of LDS (14 on a CU) and the last round counts 0.4.  In FP32, with
+// twice as many waves on a CU, it takes the longest that gives 12 waves to a
+// CU.  5x5, us per step, by rows:
+//   FP64, forty 2048 x 2048 grids     64: 268   128: 262   256: 268
+//   FP64, sixteen 2048 x 2048 grids   64: 115   128: 125
+//   FP64, sixteen 1024 x 1024 grids   16: 41.3   32: 37.5
+//   FP32, sixteen 2048 x 2048 grids   64: 69.5   128: 64.1
+//   FP32, 32 1024 x 1024 grids        32: 43.8   64: 37.5
+constexpr int kStepRows = 128;
+constexpr int kStepSlots = 14 * 256, kStepWaves32 = 12 * 256;
+
 // Item tables for a tile configuration (host copy and device copy): all
-// strips (per-grid loop and strip-only fused steps) and, with the band
-// walker, the band items of the grids it applies to (at least a strip wide
-// and a chunk and the stencil high) and the strips of the others.
+// strips (per-grid loop and strip-only steps); with the band walker, its
+// items for the grids it applies to (at least a strip wide and a chunk and
+// the stencil high) and the strips of the others; and, for a batch that
+// outgrows the L2s, the same for passes of several steps.
 hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
 {
     b->rpw = rpw;
     b->chunks = chunks;
     b->band = band;
-    int64_t strips = 0, bands = 0, rest = 0;
-    for (int gi = 0; gi < b->numGrids; gi++) {
-        BatchDev& d = b->host[gi];
-        d.stripBase = (int)strips;
-        b->strips[gi] = stripsFor(d.nx, d.ny, rpw, chunks);
-        strips += b->strips[gi];
+    auto stepItems = [&](const BatchDev& d, int n) -> int64_t {
+        const dev::StepsGrid g =
+            b->dtype == Dtype::F64
+                ? (b->H == 5 ? dev::stepsGrid<double, 5>(d.nx, d.ny, n)
+                             : dev::stepsGrid<double, 3>(d.nx, d.ny, n))
+                : (b->H == 5 ? dev::stepsGrid<float, 5>(d.nx, d.ny, n)
+                             : dev::stepsGrid<float, 3>(d.nx, d.ny, n));
+        return (int64_t)g.strips * g.bands;
+    };
+    int64_t stepBytes = 0;
+    for (const BatchDev& d : b->host)
+        if (dev::stepsApply(d.nx, d.ny))
+            stepBytes += (int64_t)d.nx * d.ny * (b->dtype == Dtype::F64 ? 8 : 4);
+    const bool passes = stepBytes > (b->H == 5 ? kStepBytes5 : kStepBytes3);
+    double least = 0;
+    for (int rows = kStepRows; rows >= 16; rows /= 2) {
+        int64_t waves = 0;
+        for (const BatchDev& d : b->host)
+            if (dev::stepsApply(d.nx, d.ny)) waves += stepItems(d, rows);
+        const double time = std::max(1.0, (double)waves / kStepSlots + 0.4) *
+                            (rows + dev::kFusedSteps * (b->V - 1) + 6);
+        if (rows == kStepRows || b->dtype == Dtype::F32 || time < least) {
+            least = time;
+            b->stepRows = rows;
+        }
+        if (b->dtype == Dtype::F32 && waves >= kStepWaves32) break;
+    }
+    int64_t n[kItemKinds] = {};
+    std::vector<int64_t> items[kItemKinds];  // of each grid
+    for (int k = 0; k < kItemKinds; k++) items[k].assign(b->numGrids, 0);
+    for (int i = 0; i < b->numGrids; i++) {
+        BatchDev& d = b->host[i];
         StencilLaunch one{};
         one.ny = one.wy1 = one.rows.rowWrap = d.ny;
         one.wx1 = d.nx;
@@ -232,46 +322,45 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
         one.rows.wrap = 1;
         one.chunks = chunks;
         d.walked = band && dev::bandApplies(one, rpw) ? 1 : 0;
-        d.bandBase = (int)bands;
-        d.restBase = (int)rest;
+        d.stepped = passes && dev::stepsApply(d.nx, d.ny) ? 1 : 0;
+        d.stripBase = (int)n[kAllStrips];
+        d.restBase = (int)n[kRestStrips];
+        d.bandBase = (int)n[kBands];
+        d.stepsBase = (int)n[kSteps];
+        d.stepsRestBase = (int)n[kStepsRest];
+        const int strips = stripsFor(d.nx, d.ny, rpw, chunks);
+        b->strips[i] = strips;
+        items[kAllStrips][i] = strips;
         if (d.walked) {
             const dev::BandGrid g = dev::bandGrid(one, rpw);
-            bands += (int64_t)g.strips * g.bands;
-        } else {
-            rest += b->strips[gi];
+            items[kBands][i] = (int64_t)g.strips * g.bands;
+        } else if (band) {
+            items[kRestStrips][i] = strips;
+        }
+        if (d.stepped) items[kSteps][i] = stepItems(d, b->stepRows);
+        else if (passes) items[kStepsRest][i] = strips;
+        for (int k = 0; k < kItemKinds; k++) {
+            n[k] += items[k][i];
+            if (n[k] > (int64_t)0x7fffffff) return hipErrorInvalidValue;
         }
     }
-    if (strips > (int64_t)0x7fffffff || bands > (int64_t)0x7fffffff ||
-        rest > (int64_t)0x7fffffff)
-        return hipErrorInvalidValue;
-    b->totalStrips = (int)strips;
-    b->totalBand = (int)bands;
-    b->totalRest = (int)rest;
-    // owning grid of every item of the three tables
-    std::vector<int> owner[3];
-    owner[0].reserve(b->totalStrips);
-    owner[1].reserve(b->totalRest);
-    owner[2].reserve(b->totalBand);
-    for (int g = 0; g < b->numGrids; g++) {
-        const BatchDev& d = b->host[g];
-        const int nBand = (g + 1 < b->numGrids ? b->host[g + 1].bandBase : b->totalBand) - d.bandBase;
-        const int nRest = (g + 1 < b->numGrids ? b->host[g + 1].restBase : b->totalRest) - d.restBase;
-        owner[0].insert(owner[0].end(), b->strips[g], g);
-        owner[1].insert(owner[1].end(), nRest, g);
-        owner[2].insert(owner[2].end(), nBand, g);
-    }
-    for (int k = 0; k < 3; k++) {
-        const size_t n = std::max<size_t>(1, owner[k].size());
-        if (n > b->itemCap[k]) {
+    std::vector<int> owner;
+    for (int k = 0; k < kItemKinds; k++) {
+        b->total[k] = (int)n[k];
+        owner.clear();
+        owner.reserve((size_t)n[k]);
+        for (int i = 0; i < b->numGrids; i++) owner.insert(owner.end(), (size_t)items[k][i], i);
+        const size_t cap = std::max<size_t>(1, owner.size());
+        if (cap > b->itemCap[k]) {
             if (b->dItemGrid[k]) (void)hipFree(b->dItemGrid[k]);
             b->dItemGrid[k] = nullptr;
             b->itemCap[k] = 0;
-            hipError_t e = hipMalloc(&b->dItemGrid[k], n * sizeof(int));
+            hipError_t e = hipMalloc(&b->dItemGrid[k], cap * sizeof(int));
             if (e != hipSuccess) return e;
-            b->itemCap[k] = n;
+            b->itemCap[k] = cap;
         }
-        if (!owner[k].empty()) {
-            hipError_t e = hipMemcpy(b->dItemGrid[k], owner[k].data(), owner[k].size() * sizeof(int),
+        if (!owner.empty()) {
+            hipError_t e = hipMemcpy(b->dItemGrid[k], owner.data(), owner.size() * sizeof(int),
                                      hipMemcpyHostToDevice);
             if (e != hipSuccess) return e;
         }
@@ -280,24 +369,39 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
                      hipMemcpyHostToDevice);
 }
 
-// One fused step at parity p: one launch over all strips, or the band walker
-// then the strips of the grids that are not walked.
+// One step at parity p: one launch over all strips, or the band walker then
+// the strips of the grids that are not walked.
 hipError_t enqueueStep(const custenBatch* b, int p, hipStream_t st)
 {
-    if (!b->band) return launchItems(b, 0, b->totalStrips, p, st, 0);
-    hipError_t e = launchItems(b, 0, b->totalBand, p, st, 2);
-    if (e == hipSuccess) e = launchItems(b, 0, b->totalRest, p, st, 1);
+    if (!b->band) return launchAll(b, kAllStrips, p, st);
+    hipError_t e = launchAll(b, kBands, p, st);
+    if (e == hipSuccess) e = launchAll(b, kRestStrips, p, st);
     return e;
 }
 
-// `steps` applies starting at parity p0.
+// kFusedSteps steps at parity p, ending on the other side (their number is
+// odd): one pass, and the single steps of the grids it leaves out.
+hipError_t enqueuePass(const custenBatch* b, int p, hipStream_t st)
+{
+    hipError_t e = launchAll(b, kSteps, p, st);
+    for (int s = 0; s < dev::kFusedSteps && e == hipSuccess; s++)
+        e = launchAll(b, kStepsRest, (p + s) & 1, st);
+    return e;
+}
+
+// `steps` applies starting at parity p0: passes of several steps, then single
+// ones, at least one, so that the other side holds the field before the last
+// step as after every run of single steps.
 hipError_t enqueueFused(const custenBatch* b, int steps, int p0, hipStream_t st)
 {
-    for (int s = 0; s < steps; s++) {
-        hipError_t e = enqueueStep(b, (p0 + s) & 1, st);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    static_assert(dev::kFusedSteps % 2 == 1, "a pass ends on the other side");
+    const int passes = b->total[kSteps] > 0 ? (steps - 1) / dev::kFusedSteps : 0;
+    int p = p0 & 1;
+    hipError_t e = hipSuccess;
+    for (int s = 0; s < passes && e == hipSuccess; s++, p ^= 1) e = enqueuePass(b, p, st);
+    for (int s = passes * dev::kFusedSteps; s < steps && e == hipSuccess; s++, p ^= 1)
+        e = enqueueStep(b, p, st);
+    return e;
 }
 
 }  // namespace
@@ -365,7 +469,6 @@ extern "C" custenBatch* custenBatchCreate(int deviceNum, int numGrids, const int
         delete b;
         return nullptr;
     }
-    b->totalStrips = (int)strips;
     if ((e = hipMalloc(&b->dGrids, sizeof(BatchDev) * numGrids)) != hipSuccess ||
         (e = configure(b, b->rpw, b->chunks, false)) != hipSuccess ||
         (e = hipMalloc(&b->dWeights, sizeof(double) * numStenHoriz * numStenVert)) != hipSuccess ||
@@ -524,7 +627,7 @@ extern "C" void custenBatchDestroy(custenBatch* b)
     for (auto& kv : b->graphs) (void)hipGraphExecDestroy(kv.second);
     for (auto& kv : b->graphDefs) (void)hipGraphDestroy(kv.second);
     if (b->dGrids) (void)hipFree(b->dGrids);
-    for (int k = 0; k < 3; k++)
+    for (int k = 0; k < kItemKinds; k++)
         if (b->dItemGrid[k]) (void)hipFree(b->dItemGrid[k]);
     if (b->dWeights) (void)hipFree(b->dWeights);
     if (b->own) (void)hipStreamDestroy(b->own);

@@ -3,8 +3,10 @@
  * counterpart in the reference, whose handles cover one grid each).
  *
  * Many independent periodic xy grids share one stencil (3x3 or 5x5 weights)
- * and are advanced together: each step is one launch over every grid, and a
- * run of steps is captured once into a HIP graph.  Per grid the results are
+ * and are advanced together: each step is one launch over every grid (three
+ * steps are, in a batch that outgrows the L2 caches, for the grids at least 128
+ * columns wide and 16 rows high), and a run of steps is captured once into a
+ * HIP graph.  Per grid the results are
  * bit-identical to cuStenCompute2DXYp followed by cuStenSwap2DXYp.
  */
 #ifndef CUSTEN_BATCH_H
@@ -23,13 +25,14 @@ custenBatch* custenBatchCreate(int deviceNum, int numGrids, const int* nx, const
                                const double* weights, int numStenHoriz, int numStenLeft,
                                int numStenVert, int numStenTop, int dtype);
 /* Apply `steps` times, swapping input and output after every apply (as
- * cuStenSwap does).  mode 0 = one launch per step for all grids (captured in
+ * cuStenSwap does); afterwards one side holds the field, the other the field
+ * before the last step.  mode 0 = one launch per step for all grids (captured in
  * a HIP graph on first use), mode 1 = plain per-grid launch loop. */
 int custenBatchRun(custenBatch* batch, int steps, int mode, hipStream_t stream);
 /* Where the current field of every grid is: 0 = dataInput[g] (before the
  * first step and after an even number of steps), 1 = dataOutput[g]. */
 int custenBatchParity(const custenBatch* batch);
-/* Tile configuration of the fused steps (results do not depend on it):
+/* Tile configuration of single fused steps (results do not depend on it):
  * band = 0: strip kernel, rowsPerWave 4 or 8 and chunks >= 1 row chunks per
  * workgroup; band = 1: band walker (chunks per band) for every grid at least
  * 128 columns wide and a chunk high, strip kernel for the rest.  Replaces the
