@@ -66,8 +66,12 @@ __host__ __device__ inline StepsGrid stepsGrid(int nx, int ny, int most)
     g.rows = (ny + g.bands - 1) / g.bands;
     return g;
 }
-// One wrap correction must do for every column and row a wave starts at.
-__host__ __device__ inline bool stepsApply(int nx, int ny) { return nx >= kTW && ny >= 16; }
+// One wrap correction must do for every column and row a wave starts at, and a
+// row's bytes for the 31 bits of a buffer's range.
+__host__ __device__ inline bool stepsApply(int nx, int ny)
+{
+    return nx >= kTW && nx < (1 << 28) && ny >= 16;
+}
 
 // K steps of wave item g of a grid (periodic, nx x ny, row stride nx).  `lds`
 // is the wave's StepsShape::ELEMS elements.
