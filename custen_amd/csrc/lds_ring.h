@@ -65,6 +65,11 @@ __device__ __forceinline__ void rowDma(__amdgpu_buffer_rsrc_t rs, Lds<char>* l, 
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LdsVoid*)l, 4, voff, soff, 0, 0);
 }
 
+__device__ __forceinline__ double rowLoad(__amdgpu_buffer_rsrc_t rs, uint32_t voff)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, 0, 0));
+}
+
 __device__ __forceinline__ void rowStore(__amdgpu_buffer_rsrc_t rs, double v, uint32_t voff,
                                          uint32_t soff)
 {

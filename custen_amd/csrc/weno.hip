@@ -1,21 +1,30 @@
 // weno.hip -- fifth-order WENO upwind advection, periodic in x and y:
 // out = u * Fx + v * Fy (cuSten/src/kernels/2d_xyADVWENO_p_kernel.cu:51-401).
 //
-// One workgroup of 256 threads covers a 64-column x 4*RPW-row tile.  The
-// tile of the advected field plus a 3-point halo on every side is staged in
-// LDS once; each lane then evaluates its column for RPW rows, reading the
-// seven-point row and column crosses from LDS and u, v from HBM.  The upwind
-// choice selects operands (no divergent branches): both signs run the same
-// flux code on differently ordered differences.
+// One workgroup of 256 threads covers a 64-column x 4*RPW-row tile.  It stages
+// the scaled differences of the advected field in LDS, in x and in y, with the
+// halo that either sign of the velocity needs, so each is taken once; a lane
+// then evaluates its column for RPW rows.  The upwind choice is a lane's address
+// and stride in LDS (the negative side reads the same differences from the other
+// end), so both signs run the same code with no selection of operands.
 //
-// The flux is evaluated operation by operation in the reference's source
-// order with contraction off; divisions are IEEE (correctly rounded), and
-// the optional single-precision squares round to float, square in float and
-// widen, as powf does on the reference's double arguments.  Results are
-// therefore bit-identical to the CPU restatement.
+// The kernel is bound by its vector instructions, so the flux is written for
+// their number: products by powers of two go into the addition that follows
+// them, and divisions run without the scaling and special cases of IEEE
+// division, which the range of the denominators makes needless; a wave that
+// meets values outside it evaluates that row again operation by operation.
+// Those two forms and the reference's source order with IEEE divisions have the
+// same bits (each shortened step is argued below), so results are bit-identical
+// to the CPU restatement.  Contraction is off; the optional single-precision
+// squares round to float, square in float and widen, as powf does on the
+// reference's double arguments.  4096 x 4096, single-precision squares: 142 us
+// at 91 % of the vector issue rate (240 instructions a point; memory alone would
+// take 100 at the copy rate); with differences and selections per lane and IEEE
+// divisions it took 192.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
+#include "lds_ring.h"  // row buffers
 #include "stencil_tile.h"
 
 #pragma clang fp contract(off)
@@ -24,7 +33,7 @@ namespace custen {
 namespace dev {
 
 constexpr int kWenoTW = 64;            // columns per tile (one per lane)
-constexpr int kWenoLD = kWenoTW + 6;   // LDS row: 3 halo columns either side
+constexpr int kWenoLX = kWenoTW + 6;   // LDS row of x differences (69 in use)
 
 template <bool SS>
 __device__ __forceinline__ double wenoSq(double d)
@@ -58,40 +67,150 @@ __device__ __forceinline__ double wenoFlux(double v1, double v2, double v3, doub
     return (phi1 * w1 + phi2 * w2) + phi3 * w3;
 }
 
-// Five upwinded differences from d[1..6], d[k] = q[c + k - 3] - q[c + k - 4]
-// scaled: u > 0 takes d[1..5], otherwise d[6..2] (2d_xyADVWENO_p_kernel.cu:288-346).
-template <bool SS>
-__device__ __forceinline__ double upwindFlux(const double (&d)[7], bool pos)
+// n / d with the bits of IEEE division, for a positive normal float d that is
+// 2^120 at most, widened: the reciprocal has 44 good bits after one Newton step
+// from the float estimate, the remainder of the quotient is exact (24 by 53
+// bits), and the quotient's last correction leaves an error of 2^-88, where no
+// quotient by a 24-bit divisor lies within 2^-78 of a rounding boundary.
+__device__ __forceinline__ double quotientF(double n, float d)
 {
-    return wenoFlux<SS>(pos ? d[1] : d[6], pos ? d[2] : d[5], pos ? d[3] : d[4],
-                        pos ? d[4] : d[3], pos ? d[5] : d[2]);
+    const double w = static_cast<double>(d);
+    double y = static_cast<double>(__builtin_amdgcn_rcpf(d));
+    y = __builtin_fma(y, __builtin_fma(-w, y, 1.0), y);
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-w, q, n), y, q);
+}
+// The steps of the GPU's IEEE division without operand scaling and fixup, which
+// leave operands alone for divisors in [2^-500, 2^500] and quotients of at least
+// 2^-400.
+__device__ __forceinline__ double recipOf(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+}
+__device__ __forceinline__ double quotient(double n, double d)
+{
+    const double y = recipOf(d);
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
+// wenoFlux with the same bits where `ok` stays true.
+// - x - 2 y and x - 4 y as one fma: the product is exact unless it overflows.
+//   Then either a sum of squares is infinite, which makes the flux NaN here, or
+//   all five differences are that large and nearly equal, and so is the flux.
+// - s + 0.25 b as one fma: the product is exact unless it is subnormal, and 1e-6
+//   is added to the sum.
+// - the squares that divide are 1e-12 at least; the upper end is tested.  The sum
+//   of the quotients is then within the range of the reciprocal's steps.
+template <bool SS>
+__device__ __forceinline__ double wenoFluxFast(double v1, double v2, double v3, double v4,
+                                               double v5, bool& ok)
+{
+    const double phi1 = ((1.0 / 3.0) * v1 - (7.0 / 6.0) * v2) + (11.0 / 6.0) * v3;
+    const double phi2 = (-(1.0 / 6.0) * v2 + (5.0 / 6.0) * v3) + (1.0 / 3.0) * v4;
+    const double phi3 = ((1.0 / 3.0) * v3 + (5.0 / 6.0) * v4) - (1.0 / 6.0) * v5;
+    const double v33 = 3.0 * v3;
+    const double s1 = __builtin_fma(0.25, wenoSq<SS>(__builtin_fma(-4.0, v2, v1) + v33),
+                                    (13.0 / 12.0) * wenoSq<SS>(__builtin_fma(-2.0, v2, v1) + v3));
+    const double s2 = __builtin_fma(0.25, wenoSq<SS>(v2 - v4),
+                                    (13.0 / 12.0) * wenoSq<SS>(__builtin_fma(-2.0, v3, v2) + v4));
+    const double s3 = __builtin_fma(0.25, wenoSq<SS>(__builtin_fma(-4.0, v4, v33) + v5),
+                                    (13.0 / 12.0) * wenoSq<SS>(__builtin_fma(-2.0, v4, v3) + v5));
+    double a1, a2, a3;
+    if constexpr (SS) {
+        const float f1 = static_cast<float>(s1 + 1e-06), f2 = static_cast<float>(s2 + 1e-06),
+                    f3 = static_cast<float>(s3 + 1e-06);
+        ok = ok && __builtin_fmaxf(__builtin_fmaxf(f1, f2), f3) <= 0x1p60f;
+        a1 = quotientF(0.1, f1 * f1);
+        a2 = quotientF(0.6, f2 * f2);
+        a3 = quotientF(0.3, f3 * f3);
+    } else {
+        const double f1 = s1 + 1e-06, f2 = s2 + 1e-06, f3 = s3 + 1e-06;
+        ok = ok && __builtin_fmax(__builtin_fmax(f1, f2), f3) <= 0x1p190;
+        a1 = quotient(0.1, f1 * f1);
+        a2 = quotient(0.6, f2 * f2);
+        a3 = quotient(0.3, f3 * f3);
+    }
+    const double sum = (a1 + a2) + a3;
+    const double y = recipOf(sum);
+    const double denom = __builtin_fma(__builtin_fma(-sum, y, 1.0), y, y);
+    const double w1 = a1 * denom, w2 = a2 * denom, w3 = a3 * denom;
+    const double flux = (phi1 * w1 + phi2 * w2) + phi3 * w3;
+    ok = ok && __builtin_fabs(flux) <= 0x1p1000;
+    return flux;
 }
 
 template <int RPW, bool SS>
-__global__ __launch_bounds__(kThreads) void wenoKernel(WenoLaunch a)
+__global__ __launch_bounds__(kThreads) void wenoKernel(WenoLaunch a, int tilesX,
+                                                         uint32_t tilesInv)
 {
     constexpr int TH = kWaves * RPW;
-    constexpr int NR = TH + 6;
-    __shared__ double tile[NR * kWenoLD];
+    // x differences: row r, column j is (q(x0 - 2 + j) - q(x0 - 3 + j)) / dx;
+    // y differences: row r is (q(y0 - 2 + r) - q(y0 - 3 + r)) / dy
+    __shared__ double diffX[TH * kWenoLX];
+    __shared__ double diffY[(TH + 5) * kWenoTW];
 
-    const int tilesX = (a.nx + kWenoTW - 1) / kWenoTW;
     const int g = xcdRemap(blockIdx.x, gridDim.x);
-    const int x0 = (g % tilesX) * kWenoTW;
-    const int y0 = (g / tilesX) * TH;
+    // g / tilesX from the rounded-down reciprocal, at most one too small
+    int tileY = (int)(((uint64_t)(uint32_t)g * tilesInv) >> 32);
+    if (g - tileY * tilesX >= tilesX) tileY++;
+    const int x0 = (g - tileY * tilesX) * kWenoTW;
+    const int y0 = tileY * TH;
     const int lane = threadIdx.x & (kLanes - 1);
-    const int wave = threadIdx.x / kLanes;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kLanes);
 
-    // LDS column j holds global column x0 - 3 + j, LDS row r region row y0 - 3 + r
-    for (int r = wave; r < NR; r += kWaves) {
-        const int sy = mapRow(a.rows, y0 - 3 + r);
-        const double* grow = a.in + (int64_t)sy * a.ldIn;
-        double* lrow = tile + r * kWenoLD;
-        lrow[3 + lane] = grow[wrapIndex(x0 + lane, a.nx)];
-        if (lane < 6) {
-            const int j = lane < 3 ? lane : kWenoTW + lane;
-            lrow[j] = grow[wrapIndex(x0 - 3 + j, a.nx)];
+    // Every load of a wave's share is issued before the first is waited for, and
+    // so are its velocities.  Rows of a tile inside the grid are buffers with
+    // their bases in scalar registers: no address arithmetic on the vector unit.
+    constexpr int PER = (TH + 5 + kWaves - 1) / kWaves;
+    const int rBegin = wave * PER, yBegin = y0 + wave * RPW;
+    double q[PER + 1], qa[RPW], qb[RPW], ta, tb, uv[RPW], vv[RPW];
+    auto row = [&](int y) { return a.in + (int64_t)mapRow(a.rows, y) * a.ldIn; };
+    // the last five x differences of the wave's rows: a lane for each
+    const int tr = min(lane / 5, RPW - 1), tc = lane - 5 * (lane / 5);
+    if (x0 >= 3 && x0 + kWenoTW + 3 <= a.nx) {
+        const uint32_t off = lane * 8u;
+#pragma unroll
+        for (int k = 0; k <= PER; k++)
+            q[k] = rowLoad(rowBuffer(row(y0 - 3 + rBegin + k) + x0), off);
+#pragma unroll
+        for (int k = 0; k < RPW; k++) {
+            const __amdgpu_buffer_rsrc_t rs = rowBuffer(row(yBegin + k) + x0 - 3);
+            qa[k] = rowLoad(rs, off + 8);
+            qb[k] = rowLoad(rs, off);
+        }
+    } else {
+        const int64_t xc = wrapIndex(x0 + lane, a.nx);
+        const int64_t xa = wrapIndex(x0 - 2 + lane, a.nx), xb = wrapIndex(x0 - 3 + lane, a.nx);
+#pragma unroll
+        for (int k = 0; k <= PER; k++) q[k] = row(y0 - 3 + rBegin + k)[xc];
+#pragma unroll
+        for (int k = 0; k < RPW; k++) {
+            qa[k] = row(yBegin + k)[xa];
+            qb[k] = row(yBegin + k)[xb];
         }
     }
+    {
+        const double* last = row(yBegin + tr);
+        ta = last[wrapIndex(x0 + kWenoTW - 2 + tc, a.nx)];
+        tb = last[wrapIndex(x0 + kWenoTW - 3 + tc, a.nx)];
+    }
+    const uint32_t here = (uint32_t)min(lane, a.nx - 1 - x0) * 8u;
+#pragma unroll
+    for (int k = 0; k < RPW; k++) {
+        const int64_t at = (int64_t)min(yBegin + k, a.ny - 1) * a.ldSide + x0;
+        uv[k] = rowLoad(rowBuffer(a.u + at), here);
+        vv[k] = rowLoad(rowBuffer(a.v + at), here);
+    }
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+        if (rBegin + k < TH + 5) diffY[(rBegin + k) * kWenoTW + lane] = (q[k + 1] - q[k]) * a.coeDy;
+#pragma unroll
+    for (int k = 0; k < RPW; k++)
+        diffX[(wave * RPW + k) * kWenoLX + lane] = (qa[k] - qb[k]) * a.coeDx;
+    if (lane < 5 * RPW) diffX[(wave * RPW + tr) * kWenoLX + kWenoTW + tc] = (ta - tb) * a.coeDx;
     __syncthreads();
 
     const int x = x0 + lane;
@@ -101,19 +220,24 @@ __global__ __launch_bounds__(kThreads) void wenoKernel(WenoLaunch a)
         const int ly = wave * RPW + r;
         const int y = y0 + ly;
         if (y >= a.ny) break;
-        const double* c = tile + (ly + 3) * kWenoLD + 3 + lane;
-        double dx[7], dy[7];
-#pragma unroll
-        for (int k = 1; k < 7; k++) {
-            dx[k] = (c[k - 3] - c[k - 4]) * a.coeDx;
-            dy[k] = (c[(k - 3) * kWenoLD] - c[(k - 4) * kWenoLD]) * a.coeDy;
+        // the middle one of the five differences, and the way to the others
+        const bool px = uv[r] > 0.0, py = vv[r] > 0.0;
+        const double* mx = diffX + ly * kWenoLX + lane + (px ? 2 : 3);
+        const double* my = diffY + (ly + (py ? 2 : 3)) * kWenoTW + lane;
+        const int sx = px ? 1 : -1, sy = py ? kWenoTW : -kWenoTW;
+        double dx[5] = {mx[-2 * sx], mx[-sx], mx[0], mx[sx], mx[2 * sx]};
+        double dy[5] = {my[-2 * sy], my[-sy], my[0], my[sy], my[2 * sy]};
+        bool ok = true;
+        double fx = wenoFluxFast<SS>(dx[0], dx[1], dx[2], dx[3], dx[4], ok);
+        double fy = wenoFluxFast<SS>(dy[0], dy[1], dy[2], dy[3], dy[4], ok);
+        if (__builtin_expect(__ballot(!ok) != 0, 0)) {
+            // (taken from here on, so that it is not computed beside the other)
+            __asm__ __volatile__("" : "+v"(dx[0]), "+v"(dx[1]), "+v"(dx[2]), "+v"(dx[3]), "+v"(dx[4]));
+            __asm__ __volatile__("" : "+v"(dy[0]), "+v"(dy[1]), "+v"(dy[2]), "+v"(dy[3]), "+v"(dy[4]));
+            fx = wenoFlux<SS>(dx[0], dx[1], dx[2], dx[3], dx[4]);
+            fy = wenoFlux<SS>(dy[0], dy[1], dy[2], dy[3], dy[4]);
         }
-        const int64_t is = (int64_t)y * a.ldSide + x;
-        const double uu = a.u[is];
-        const double vv = a.v[is];
-        const double fx = upwindFlux<SS>(dx, uu > 0.0);
-        const double fy = upwindFlux<SS>(dy, vv > 0.0);
-        __builtin_nontemporal_store(uu * fx + vv * fy, a.out + (int64_t)y * a.ldOut + x);
+        __builtin_nontemporal_store(uv[r] * fx + vv[r] * fy, a.out + (int64_t)y * a.ldOut + x);
     }
 }
 
@@ -121,31 +245,32 @@ template <int RPW>
 hipError_t launchWenoRpw(const WenoLaunch& w, hipStream_t st)
 {
     constexpr int TH = kWaves * RPW;
-    const int64_t tiles = (int64_t)((w.nx + kWenoTW - 1) / kWenoTW) * ((w.ny + TH - 1) / TH);
+    const int64_t tilesX = (w.nx + kWenoTW - 1) / kWenoTW;
+    const int64_t tiles = tilesX * ((w.ny + TH - 1) / TH);
     if (tiles > 0x7fffffff) return hipErrorInvalidValue;
-    if (w.singleSquares)
-        hipLaunchKernelGGL((wenoKernel<RPW, true>), dim3((unsigned)tiles), dim3(kThreads), 0, st, w);
-    else
-        hipLaunchKernelGGL((wenoKernel<RPW, false>), dim3((unsigned)tiles), dim3(kThreads), 0, st, w);
+    // (2^32 - 1) / tilesX: also fits where tilesX is 1
+    const uint32_t inv = 0xffffffffu / (uint32_t)tilesX;
+    auto* kernel = w.singleSquares ? wenoKernel<RPW, true> : wenoKernel<RPW, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(kThreads), 0, st, w, (int)tilesX, inv);
     return hipGetLastError();
 }
 
 }  // namespace dev
 
-// 8 rows per wave unless 4 is asked for: measured faster at 8192^2 with both
-// treatments of the squares (the kernel is VALU-bound; taller tiles re-read
-// fewer halo rows and give each wave more independent points).
+// 4 rows per wave unless 8 is asked for: the same time at 4096 x 4096 (147 and
+// 146 us) and less where there are few tiles (300 x 500: 6.5 and 10.0 us).
 int wenoLdsBytes(int rowsPerWave)
 {
-    const int rpw = rowsPerWave == 4 ? 4 : 8;
-    return (dev::kWaves * rpw + 6) * dev::kWenoLD * (int)sizeof(double);
+    const int rpw = rowsPerWave == 8 ? 8 : 4;
+    const int rows = dev::kWaves * rpw;
+    return (rows * dev::kWenoLX + (rows + 5) * dev::kWenoTW) * (int)sizeof(double);
 }
 
 hipError_t launchWeno(const WenoLaunch& w, hipStream_t st)
 {
     if (w.nx < 1 || w.ny < 1) return hipSuccess;
-    if (w.rowsPerWave == 4) return dev::launchWenoRpw<4>(w, st);
-    return dev::launchWenoRpw<8>(w, st);
+    if (w.rowsPerWave == 8) return dev::launchWenoRpw<8>(w, st);
+    return dev::launchWenoRpw<4>(w, st);
 }
 
 }  // namespace custen
