@@ -265,20 +265,35 @@ public:
         return hipSuccess;
     }
 
-    // k steps of all resident requests as one launch: the step kernels of the
-    // k steps are captured once into a HIP graph and replayed while the
-    // resident set (and so the descriptors) and k stay the same.  The
-    // kernels use a step number only modulo 3 relative to each request's
-    // admission (which field buffer is current), so a graph serves every
-    // batch whose first step has the residue it was captured at.  Replaying
-    // one graph costs the host one launch instead of 4 k + 1.  Consecutive batches alternate between two
-    // graphs: launching a graph whose previous launch is still running makes
-    // the host wait for it.
+    // k steps of all resident requests.  Batches that repeat are captured into
+    // a HIP graph and replayed while the resident set (and so the
+    // descriptors) and k stay the same: one launch for the host instead of
+    // 4 k + 1.  The kernels use a step number only modulo 3 relative to each
+    // request's admission (which field buffer is current), so a graph serves
+    // every batch whose first step has the residue it was captured at; with
+    // batches of a multiple of 3 steps that is every batch.  Instantiating a
+    // graph and launching it for the first time costs the host 0.5-1.3 ms, ten
+    // times what 37 launches do, so a batch is captured only after
+    // kCaptureAfter like it.  (With batches of 8 steps and no such rule every
+    // batch was captured: four lanes of 64 to 160 points a side were held to
+    // the host's pace, 109 ms for 2000 steps where it is 95 now.)  Consecutive
+    // batches alternate between two graphs: launching a graph whose previous launch is
+    // still running makes the host wait for it.
     hipError_t stepBatch(hipStream_t st, int k)
     {
         if (active_.empty() || k <= 0) return hipSuccess;
         hipError_t e;
         if (dirty_ && (e = upload(st)) != hipSuccess) return e;
+        const bool again = lastK_ == k && lastVersion_ == version_ && lastResidue_ == step_ % 3;
+        repeats_ = again ? repeats_ + 1 : 0;
+        lastK_ = k;
+        lastVersion_ = version_;
+        lastResidue_ = (step_ + k) % 3;  // of the next batch, if its steps follow
+        if (repeats_ < kCaptureAfter || k % 3 != 0) {
+            if ((e = launchSteps(st, step_, k)) != hipSuccess) return e;
+            step_ += k;
+            return hipSuccess;
+        }
         BatchGraph& g = graphs_[launches_ & 1];
         if (!g.exec || g.k != k || g.version != version_ || g.parity != step_ % 3) {
             if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -427,6 +442,10 @@ private:
     };
     BatchGraph graphs_[2];
     uint64_t launches_ = 0;
+    // the last batch, and how many like it went before
+    int lastK_ = 0, lastResidue_ = 0, repeats_ = 0;
+    uint64_t lastVersion_ = 0;
+    static constexpr int kCaptureAfter = 4;
     uint64_t version_ = 0;  // bumped by every descriptor upload
 };
 
@@ -883,8 +902,10 @@ struct custenCHServer {
 
 namespace {
 
-// Steps a lane enqueues at once (fewer if a request finishes earlier).
-constexpr int kLaneBatch = 8;
+// Steps a lane enqueues at once (fewer if a request finishes earlier); a
+// multiple of the three field buffers, so that every batch starts at the same
+// one and captured batches fit (see CHEngine::stepBatch).
+constexpr int kLaneBatch = 9;
 // Finished results kept in pinned memory up to this many bytes (the
 // environment variable CUSTEN_CH_PINNED_RESULT_BYTES, read when a server is
 // created, overrides it); later ones move to pageable memory once their copy
