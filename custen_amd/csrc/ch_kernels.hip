@@ -263,11 +263,19 @@ __global__ __launch_bounds__(256) void transposeKernel(const CHDesc* __restrict_
 // every load and store is unconditional (row indices past the sweep are
 // clamped to a valid row and their values unused), so the wait counts the
 // compiler computes are exact and no wait drains the loads still in flight.
-// Steps that do not fit whole are done one row at a time after the loop.
+// Rows that do not fill a step are done one at a time after the loop, from
+// registers that were loaded before it.
 // The factored rows settle into a constant run (chConstantRuns); the steps
 // inside it run as a loop of their own with the run's values as uniform
 // constants and no ring, and divide in two operations when the host has
 // certified the run's pivot (chDivCertified).
+//
+// One wave to a CU at 1024 columns: the time is the wave's own instructions,
+// 10 a row forward and 6 backward at about 5 clocks each, of which two export a
+// row at 12, and the latencies that it meets alone.  1024 x 1024: 52.5 us, of 57.5
+// before the loads ahead carried over from the one loop to the next, the rows
+// left and the rows of the ends were loaded ahead, and the upper limit of the
+// two-operation division was found not to need a test in each row.
 // ---------------------------------------------------------------------------
 constexpr int SR = 16;  // rows per step (settleStep takes 16)
 
@@ -293,6 +301,14 @@ __device__ __forceinline__ double divByRecip(double n, double d, double y)
     double q = n * y;
     q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
     return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+
+// v of lane i (the same for all lanes).
+__device__ __forceinline__ double laneValue(double v, int i)
+{
+    const u32x2 p = __builtin_bit_cast(u32x2, v);
+    return __builtin_bit_cast(double, u32x2{(uint32_t)__builtin_amdgcn_readlane((int)p.x, i),
+                                            (uint32_t)__builtin_amdgcn_readlane((int)p.y, i)});
 }
 
 // One wait for a whole step of rows: the empty statement takes all SR
@@ -322,7 +338,8 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
     const int colRaw = (item - D.colBase) * kCHColBlock + lane;
     const bool live = colRaw < n;
     const int col = live ? colRaw : n - 1;
-    gdouble* __restrict__ base = (gdouble*)(which ? D.X : D.Y);
+    // (not restrict: the steps go to the same rows through buffers)
+    gdouble* base = (gdouble*)(which ? D.X : D.Y);
     const int64_t s = n;
     const gdouble* __restrict__ ds = (const gdouble*)D.fac;
     const gdouble* __restrict__ dl = ds + m;
@@ -358,10 +375,20 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
     const double k0 = ds[kf], k1 = dl[kf], k2 = dd[kf], ky = divRecip(k2);
     const double ku = du[kb], kw = dw[kb];
 
+    // rows left after the whole steps: the last of the forward sweep and the
+    // first of the grid for the backward one
+    const int rem = (m - 2) - nFull * SR;
+    const double duEnd = du[m - 2];
+    const double endRow2 = at(n - 2), endRow1 = at(n - 1);
+
     // ---- forward substitution: rows 0 and 1, then rows 2 .. m-1 in steps
-    double b2 = at(0) / dd[0];
+    const double row0 = at(0), row1 = at(1);
+    double tail[SR];  // the rows left, loaded ahead (past them, the last one)
+#pragma unroll
+    for (int k = 0; k < SR; k++) tail[k] = at(min(m - rem + k, m - 1));
+    double b2 = row0 / dd[0];
     at(0) = b2;
-    double b1 = (at(1) - dl[1] * b2) / dd[1];
+    double b1 = (row1 - dl[1] * b2) / dd[1];
     at(1) = b1;
     if (nFull > 0) {
         // rows 2 + j SR + k of step j (steps past the sweep: the last one)
@@ -442,11 +469,14 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 if constexpr (decltype(fast)::value) v = __builtin_fma(num, ky, num * kz);
                 else v = divByRecip(num, k2, ky);
                 nmin = __builtin_fmin(nmin, __builtin_fabs(num));
-                nmax = __builtin_fmax(nmax, __builtin_fabs(num));
+                if constexpr (!decltype(fast)::value) nmax = __builtin_fmax(nmax, __builtin_fabs(num));
                 store(out, k, v);
                 b2 = b1;
                 b1 = v;
             }
+            // (the two-operation division has no upper limit short of Inf and
+            // NaN, and those stay in the recurrence to the end of the step)
+            if constexpr (decltype(fast)::value) nmax = __builtin_fabs(b1) <= 0x1.fffffffffffffp1023 ? 0.0 : 0x1p1000;
             if (__builtin_expect(!(nmin >= 0x1p-900 && nmax <= 0x1p900 && ky != 0.0), 0)) {
                 b2 = b2s;
                 b1 = b1s;
@@ -459,17 +489,19 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 }
             }
         };
-        // steps [0, jc) read the ring, steps [jc, nFull) start at or after cfw
-        const int jc = min((cfw - 2 + SR - 1) / SR, nFull);
+        // steps [0, jc) read the ring, steps [jc, nFull) start at or after cfw;
+        // jc is a multiple of three, where the buffers are back in their
+        // places, so that the steps loaded ahead carry over
+        const int jc = min(((cfw - 2 + SR - 1) / SR + 2) / 3 * 3, nFull);
         double bufA[SR], bufB[SR], bufC[SR];
         __amdgpu_buffer_rsrc_t rA, rB, rC;  // the rows of the steps in bufA, bufB, bufC
+        loadStep(bufA, rA, 0);
+        loadStep(bufB, rB, 1);
         if (jc > 0) {
             {
                 const int r0 = diagRow(0);
                 stageDiag(0, ds[r0], dl[r0], dd[r0]);
             }
-            loadStep(bufA, rA, 0);
-            loadStep(bufB, rB, 1);
             int j = 0;
             for (; j + 3 <= jc; j += 3) {
                 step(j, bufA, bufC, rA, rC);
@@ -480,8 +512,6 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             if (j < jc) step(j++, bufB, bufA, rB, rA);
         }
         auto constSteps = [&](auto fast) {
-            loadStep(bufA, rA, jc);
-            loadStep(bufB, rB, jc + 1);
             int j = jc;
             for (; j + 3 <= nFull; j += 3) {
                 stepK(fast, j, bufA, bufC, rA, rC);
@@ -492,7 +522,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             if (j < nFull) stepK(fast, j++, bufB, bufA, rB, rA);
         };
         if (jc < nFull) {
-            if (D.fastDiv) {
+            if (D.fastDiv && k1 != 0.0) {
                 kz = __builtin_fma(-k2, ky, 1.0) / k2;
                 constSteps(std::true_type{});
             } else {
@@ -500,22 +530,37 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             }
         }
     }
-    // rows left after the whole steps, one at a time
-    for (int i = 2 + nFull * SR; i < m; i++) {
-        const double t = at(i) - ds[i] * b2;
-        const double v = (t - dl[i] * b1) / dd[i];
-        at(i) = v;
-        b2 = b1;
-        b1 = v;
+    if (m - rem >= cfw) {
+#pragma unroll
+        for (int k = 0; k < SR; k++) {
+            if (k >= rem) break;
+            const double t = tail[k] - k0 * b2;
+            const double v = (t - k1 * b1) / k2;
+            at(m - rem + k) = v;
+            b2 = b1;
+            b1 = v;
+        }
+    } else {
+        for (int i = m - rem; i < m; i++) {
+            const double t = at(i) - ds[i] * b2;
+            const double v = (t - dl[i] * b1) / dd[i];
+            at(i) = v;
+            b2 = b1;
+            b1 = v;
+        }
     }
 
     // ---- backward substitution: b1 = x[m-1], b2 = b[m-2]; then rows m-3
     // down to 0 in steps
     const double xm1 = b1;
     double a1 = b1;
-    double a0 = b2 - du[m - 2] * a1;
+    double a0 = b2 - duEnd * a1;
     at(m - 2) = a0;
     const double xm2 = a0;
+    // the rows left of this sweep, 0 .. rem - 1 (past them, row 0)
+    double tailU = du[min(lane, SR - 1)], tailW = dw[min(lane, SR - 1)];
+#pragma unroll
+    for (int k = 0; k < SR; k++) tail[k] = at(max(rem - 1 - k, 0));
     if (nFull > 0) {
         // step j holds rows m-3 - j SR - k; row k of the step sits at offset
         // SR-1-k above the step's lowest row m-3 - j SR - (SR-1)
@@ -541,7 +586,9 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         // steps [0, jcb) lie in the constant run (their lowest row is at or
         // above cbw), steps [jcb, nFull) read the ring
         const int lowest0 = m - 3 - (SR - 1);
-        const int jcb = lowest0 >= cbw ? min((lowest0 - cbw) / SR + 1, nFull) : 0;
+        // (a multiple of three, as jc, or all of them)
+        int jcb = lowest0 >= cbw ? min((lowest0 - cbw) / SR + 1, nFull) : 0;
+        if (jcb < nFull) jcb -= jcb % 3;
         auto step = [&](int j, const double (&cur)[SR], double (&ahead)[SR],
                         const __amdgpu_buffer_rsrc_t& out, __amdgpu_buffer_rsrc_t& outAhead) {
             const int rd = diagRow(j + 1);
@@ -574,9 +621,9 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         };
         double bufA[SR], bufB[SR], bufC[SR];
         __amdgpu_buffer_rsrc_t rA, rB, rC;  // the rows of the steps in bufA, bufB, bufC
+        loadStep(bufA, rA, 0);
+        loadStep(bufB, rB, 1);
         if (jcb > 0) {
-            loadStep(bufA, rA, 0);
-            loadStep(bufB, rB, 1);
             int j = 0;
             for (; j + 3 <= jcb; j += 3) {
                 stepK(j, bufA, bufC, rA, rC);
@@ -591,8 +638,6 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 const int r0 = diagRow(jcb);
                 stageDiag(0, du[r0], dw[r0]);
             }
-            loadStep(bufA, rA, jcb);
-            loadStep(bufB, rB, jcb + 1);
             int j = jcb;
             for (; j + 3 <= nFull; j += 3) {
                 step(j, bufA, bufC, rA, rC);
@@ -603,9 +648,13 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             if (j < nFull) step(j++, bufB, bufA, rB, rA);
         }
     }
-    for (int i = m - 3 - nFull * SR; i >= 0; i--) {
-        const double t = at(i) - du[i] * a0;
-        const double v = t - dw[i] * a1;
+    static_assert(SR <= kCHColBlock, "a lane for each row left");
+#pragma unroll
+    for (int k = 0; k < SR; k++) {
+        if (k >= rem) break;
+        const int i = rem - 1 - k;
+        const double t = tail[k] - laneValue(tailU, i) * a0;
+        const double v = t - laneValue(tailW, i) * a1;
         at(i) = v;
         a1 = a0;
         a0 = v;
@@ -613,8 +662,8 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
     if (!live) return;
     // solveEnd: a0 = x[0], a1 = x[1]
     gdouble* __restrict__ Xc = base + col;
-    const double e2 = Xc[(n - 2) * s] - (D.e * a0 + D.a * xm2 + D.b * xm1);
-    const double e1 = Xc[(n - 1) * s] - (D.d * a0 + D.e * a1 + D.a * xm1);
+    const double e2 = endRow2 - (D.e * a0 + D.a * xm2 + D.b * xm1);
+    const double e1 = endRow1 - (D.d * a0 + D.e * a1 + D.a * xm1);
     Xc[(n - 2) * s] = D.omega[0] * e2 + D.omega[1] * e1;
     Xc[(n - 1) * s] = D.omega[2] * e2 + D.omega[3] * e1;
 }
