@@ -95,6 +95,8 @@ hipError_t builtinFunctionAddress(Builtin b, void** addr);
 int stencilLdsBytes(Dtype dt, int H, int V, int rowsPerWave);
 // LDS bytes of one band-walker workgroup (one wave).
 int stencilBandLdsBytes(Dtype dt, int H, int V, int rowsPerWave);
+// chunks per band (4 rows each) with which a shape that can streams its rows; 0: none
+int stencilRowsChunks(Dtype dt, int H, int V, int nx, int ny);
 
 // WENO5 upwind advection over a region of rows [0, ny), periodic in x: out =
 // u * Fx + v * Fy.  `in` rows are addressed through `rows` (the kernel reads

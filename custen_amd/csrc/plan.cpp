@@ -818,6 +818,8 @@ void computeCommon(cuSten_t* h, bool offload, const char* fn)
                          {TuneVal{4, 2, 2, 1}, TuneVal{4, 4, 2, 1}, TuneVal{4, 8, 2, 1},
                           TuneVal{8, 1, 2, 1}, TuneVal{8, 2, 2, 1}, TuneVal{8, 4, 2, 1}})
                         cands.push_back(b);
+                    if (const int c = p->fun ? 0 : stencilRowsChunks(p->dtype, p->H, p->V, h->nx, h->ny))
+                        cands.push_back({4, c, 2, 1});
                 }
                 auto run = [&](const TuneVal& c) {
                     Plan tmp = *p;

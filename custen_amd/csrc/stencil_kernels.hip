@@ -19,6 +19,7 @@
 #include "kernels.h"
 #include "stencil_band.h"
 #include "stencil_body.h"
+#include "stencil_rows.h"
 #include "stencil_tile.h"
 
 #pragma clang fp contract(off)
@@ -420,6 +421,15 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
     if constexpr (bandShape && CPL == 2 && (RPW == 4 || RPW == 8)) {
         if (s.band && dev::bandApplies(s, RPW)) {
             const dev::BandGrid g = dev::bandGrid(s, RPW);
+            if constexpr (dev::kStreamRows<T, H, V>) {
+                if (s.chunks * RPW >= dev::kStreamBand) {
+                    const int64_t rowWaves = (int64_t)g.strips * dev::rowsBands(g, s.chunks * RPW);
+                    if (rowWaves > 0x7fffffff) return hipErrorInvalidValue;
+                    hipLaunchKernelGGL((dev::stencilRows<H, V>), dim3((unsigned)rowWaves),
+                                       dim3(dev::kLanes), 0, st, s);
+                    return hipGetLastError();
+                }
+            }
             const int64_t waves = (int64_t)g.strips * g.bands;
             if (waves > 0x7fffffff) return hipErrorInvalidValue;
             hipLaunchKernelGGL((dev::stencilBand<T, H, V, RPW, X>), dim3((unsigned)waves),
@@ -543,6 +553,35 @@ int stencilLdsBytes(Dtype dt, int H, int V, int rowsPerWave)
     return es * (dev::kWaves * rpw + V - 1) * dev::ldsRowLength(H);
 }
 
+// Rows stream in long bands only: one row costs a wave the same whether its
+// sums are stored or not, a SIMD takes its waves in turn, and V rows are taken
+// at a time.  So a launch costs waves per SIMD (a lone one as much as 1.4)
+// times rows of a band, in groups of V, at kUnit us each, against kPoint us a
+// point for the chunks (both measured, 4096 x 4096, random data; on the way the
+// clock falls with the power that dense FP64 FMAs draw).  Returns the chunks of
+// 4 rows of the best band, or 0 where the chunked walker is faster.
+//   9x9, us, chunks against rows: 2048^2: 28.5, 28.1   3001 x 2999: 51.4, 41.7
+//   4096^2: 85.7, 67.3   8192^2: 315, 262
+//   7x7: 2048^2: 16.1, 21.7   3001 x 2999: 38.3, 30.4   4096^2: 58.3, 49.3
+int stencilRowsChunks(Dtype dt, int H, int V, int nx, int ny)
+{
+    if (dt != Dtype::F64 || H != V || (H != 7 && H != 9)) return 0;
+    const double kUnit = H == 9 ? 0.455 : 0.36, kPoint = H == 9 ? 5.3e-6 : 3.6e-6;
+    const int64_t strips = (nx + dev::kTW - 1) / dev::kTW;
+    double least = kPoint * nx * ny;
+    int best = 0;
+    for (int rows = dev::kStreamBand; rows <= 192; rows += 4) {
+        const int64_t waves = strips * ((ny + rows - 1) / rows), perSimd = (waves + 1023) / 1024;
+        const int groups = (rows + V - 1 + V - 1) / V;
+        const double time = kUnit * (perSimd == 1 ? 1.4 : (double)perSimd) * groups * V;
+        if (time < least) {
+            least = time;
+            best = rows / 4;
+        }
+    }
+    return best;
+}
+
 int stencilBandLdsBytes(Dtype dt, int H, int V, int rowsPerWave)
 {
     const int rpw = rowsPerWave == 8 ? 8 : 4;
@@ -562,7 +601,10 @@ hipError_t launchStencil(const StencilLaunch& in, hipStream_t st)
     if (s.rowsPerWave == 0 && s.chunks == 0 && s.colsPerLane == 0 && !s.band) {
         s.band = 1;
         s.rowsPerWave = 4;
-        s.chunks = (int64_t)s.nx * s.ny >= kLongBandPoints ? 2 : 1;
+        s.chunks = s.xform == Xform::Identity
+                       ? stencilRowsChunks(s.dtype, s.H, s.V, s.nx, s.ny)
+                       : 0;
+        if (s.chunks == 0) s.chunks = (int64_t)s.nx * s.ny >= kLongBandPoints ? 2 : 1;
     }
     if (s.colsPerLane != 1) s.colsPerLane = 2;
     if (s.colsPerLane == 1) {
