@@ -198,7 +198,10 @@ __global__ __launch_bounds__(256) void rhsKernel(const CHDesc* __restrict__ desc
 // column solveFull of the x-direction solves applied (serialCahnADI.c:661-678):
 // y_j -= inv1[j] y~2 + inv2[j] y~1, j < n-2.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void transposeKernel(const CHDesc* __restrict__ descs, int count)
+// One tile to a CU at n = 1024: its latencies are met by more waves (256 threads:
+// 8.8 us, 512: 8.2; 4096: 45.6 and 46.4).
+constexpr int kTrThreads = 512;
+__global__ __launch_bounds__(kTrThreads) void transposeKernel(const CHDesc* __restrict__ descs, int count)
 {
     __shared__ double t[kCHTr][kCHTr + 1];
     const int item = blockIdx.x;
@@ -217,21 +220,21 @@ __global__ __launch_bounds__(256) void transposeKernel(const CHDesc* __restrict_
     const gdouble* inv2 = inv1 + m;
     // all loads first (points past the grid repeat its last row or column),
     // then the corrections and the guarded LDS writes
-    constexpr int kRowsPerWave = kCHTr / 4;
+    constexpr int kWavesTr = kTrThreads / 64, kRowsPerWave = kCHTr / kWavesTr;
     const int cc = min(c, n - 1);
     const double e2 = src[(int64_t)(n - 2) * n + cc];
     const double e1 = src[(int64_t)(n - 1) * n + cc];
     double v[kRowsPerWave], i1[kRowsPerWave], i2[kRowsPerWave];
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; i++) {
-        const int row = R0 + wave + 4 * i;
+        const int row = R0 + wave + kWavesTr * i;
         v[i] = src[(int64_t)min(row, n - 1) * n + cc];
         i1[i] = inv1[min(row, m - 1)];
         i2[i] = inv2[min(row, m - 1)];
     }
 #pragma unroll
     for (int i = 0; i < kRowsPerWave; i++) {
-        const int k = wave + 4 * i;
+        const int k = wave + kWavesTr * i;
         const int row = R0 + k;
         if (row < n && c < n) {
             double w = v[i];
@@ -241,7 +244,7 @@ __global__ __launch_bounds__(256) void transposeKernel(const CHDesc* __restrict_
     }
     __syncthreads();
 #pragma unroll 4
-    for (int k = wave; k < kCHTr; k += 4) {
+    for (int k = wave; k < kCHTr; k += kWavesTr) {
         const int row = C0 + k;  // destination row = source column
         const int col = R0 + lane;
         if (row < n && col < n) dst[(int64_t)row * n + col] = t[lane][k];
@@ -272,36 +275,46 @@ __global__ __launch_bounds__(256) void transposeKernel(const CHDesc* __restrict_
 //
 // One wave to a CU at 1024 columns: the time is the wave's own instructions,
 // 10 a row forward and 6 backward at about 5 clocks each, of which two export a
-// row at 12, and the latencies that it meets alone.  1024 x 1024: 52.5 us, of 57.5
-// before the loads ahead carried over from the one loop to the next, the rows
-// left and the rows of the ends were loaded ahead, and the upper limit of the
-// two-operation division was found not to need a test in each row.
+// row at 12, and the latencies that it meets alone; rows outside the constant
+// runs take 16 and 8.  1024 x 1024: 50.4 us, of 57.5 before the loads ahead carried
+// over from the one loop to the next, the rows left and the rows of the ends
+// were loaded ahead, the upper limit of the short divisions was found not to
+// need a test in each row, and the ring was read a group ahead (256 x 256, whose
+// factors never settle: 20.9 us, of 25.3; 4096 x 4096: 255, of 290).
 // ---------------------------------------------------------------------------
 constexpr int SR = 16;  // rows per step (settleStep takes 16)
 
-// Reciprocal of a diagonal entry for the division below: RN(1/d) when
-// 2^-60 <= |d| <= 2^60, else 0 (the row then divides with IEEE division).
+// RN(1/d) for the two-operation division when 2^-60 <= |d| <= 2^60, else 0 (the
+// row then divides with IEEE division).
 __device__ __forceinline__ double divRecip(double d)
 {
     const double ad = __builtin_fabs(d);
     return (ad >= 0x1p-60 && ad <= 0x1p60) ? 1.0 / d : 0.0;
 }
 
-// n / d, correctly rounded, with y = RN(1/d) precomputed (all columns of a
-// request share the matrix, so y is computed once per row, off the
-// recurrence's critical path).  q0 = RN(n y) and two corrections
-// q <- RN(q + RN(n - d q) y) (each remainder exact by fma) give RN(n / d)
-// (Markstein's theorem: the first correction makes q faithful, the second
-// rounds it correctly); the dependent chain is five operations against the
-// eleven of the scaled IEEE sequence.  The preconditions (no overflow and no
-// subnormal intermediate) hold for 2^-900 <= |n| <= 2^900 and the range of d
-// in divRecip (y != 0).
+// The GPU's IEEE division (reciprocal estimate, two Newton steps, quotient,
+// remainder, one correction) without its operand scaling and fixup, which leave
+// operands alone in the range below; the reciprocal comes once a row, off the
+// recurrence's critical path, as all columns of a request share the matrix.  The
+// dependent chain is three operations against eleven.  The preconditions (no
+// subnormal intermediate, 2^-60 <= |d| <= 2^60, where divRecip is not 0) hold for
+// |n| >= 2^-900; infinities and NaN need IEEE division.
+__device__ __forceinline__ double divRecip2(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    const double ad = __builtin_fabs(d);
+    return (ad >= 0x1p-60 && ad <= 0x1p60) ? y : 0.0;
+}
 __device__ __forceinline__ double divByRecip(double n, double d, double y)
 {
-    double q = n * y;
-    q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
+    const double q = n * y;
     return __builtin_fma(__builtin_fma(-d, q, n), y, q);
 }
+// An infinity or NaN stays in the recurrence to the end of a step, where its
+// last value shows it (the factors of the value before are not 0).
+__device__ __forceinline__ bool isFinite(double v) { return __builtin_fabs(v) < __builtin_inf(); }
 
 // v of lane i (the same for all lanes).
 __device__ __forceinline__ double laneValue(double v, int i)
@@ -310,6 +323,21 @@ __device__ __forceinline__ double laneValue(double v, int i)
     return __builtin_bit_cast(double, u32x2{(uint32_t)__builtin_amdgcn_readlane((int)p.x, i),
                                             (uint32_t)__builtin_amdgcn_readlane((int)p.y, i)});
 }
+
+// Four rows, from row k0 on, of A arrays of a slot of the diagonals' ring.  They
+// are read a group ahead of the rows that use them: the compiler issues a read
+// where it is needed, which cost the wave two LDS latencies in four rows.
+template <int A>
+struct RingRows {
+    double v[A][4];
+    __device__ __forceinline__ RingRows(const double (&slot)[4][kCHColBlock], int k0)
+    {
+#pragma unroll
+        for (int a = 0; a < A; a++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[a][i] = slot[a][k0 + i];
+    }
+};
 
 // One wait for a whole step of rows: the empty statement takes all SR
 // values as operands, so the compiler waits once for the loads that fill
@@ -384,8 +412,11 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
     // ---- forward substitution: rows 0 and 1, then rows 2 .. m-1 in steps
     const double row0 = at(0), row1 = at(1);
     double tail[SR];  // the rows left, loaded ahead (past them, the last one)
+    auto loadTail = [&]() {
 #pragma unroll
-    for (int k = 0; k < SR; k++) tail[k] = at(min(m - rem + k, m - 1));
+        for (int k = 0; k < SR; k++) tail[k] = at(min(m - rem + k, m - 1));
+    };
+    if (nFull == 0) loadTail();
     double b2 = row0 / dd[0];
     at(0) = b2;
     double b1 = (row1 - dl[1] * b2) / dd[1];
@@ -402,15 +433,16 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
 #pragma unroll
             for (int k = 0; k < SR; k++) buf[k] = load(p, k);
         };
-        // every row of the staged step has a reciprocal (uniform)
+        // every row of the staged step has a reciprocal, and a factor of the
+        // row before (uniform)
         bool recips = true;
         auto stageDiag = [&](int slot, double p0, double p1, double p2) {
-            const double y = divRecip(p2);
+            const double y = divRecip2(p2);
             sd[slot][0][lane] = p0;
             sd[slot][1][lane] = p1;
             sd[slot][2][lane] = p2;
             sd[slot][3][lane] = y;
-            recips = __all(y != 0.0);
+            recips = __all(y != 0.0 && p1 != 0.0);
         };
         auto diagRow = [&](int j) { return min(2 + j * SR + min(lane, SR - 1), m - 1); };
         // step j: diagonals of step j+1 and the column rows of step j+2 are
@@ -420,25 +452,33 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             const int rd = diagRow(j + 1);
             const double p0 = ds[rd], p1 = dl[rd], p2 = dd[rd];
             loadStep(ahead, outAhead, j + 2);
-            settleStep(cur);
             const int slot = j & 1;
-            double nmin = 0x1p900, nmax = 0x1p-900;
+            RingRows<4> ahead0(sd[slot], 0);
+            settleStep(cur);
+            double nmin = 0x1p900;
             const double b2s = b2, b1s = b1;
 #pragma unroll
-            for (int k = 0; k < SR; k++) {
-                const double t = cur[k] - sd[slot][0][k] * b2;
-                const double num = t - sd[slot][1][k] * b1;
-                const double v = divByRecip(num, sd[slot][2][k], sd[slot][3][k]);
-                nmin = __builtin_fmin(nmin, __builtin_fabs(num));
-                nmax = __builtin_fmax(nmax, __builtin_fabs(num));
-                store(out, k, v);
-                b2 = b1;
-                b1 = v;
+            for (int q = 0; q < SR / 4; q++) {
+                RingRows<4> f = ahead0;
+                if (q + 1 < SR / 4) ahead0 = RingRows<4>(sd[slot], 4 * (q + 1));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int k = 4 * q + i;
+                    const double t = cur[k] - f.v[0][i] * b2;
+                    const double num = t - f.v[1][i] * b1;
+                    const double v = divByRecip(num, f.v[2][i], f.v[3][i]);
+                    nmin = __builtin_fmin(nmin, __builtin_fabs(num));
+                    store(out, k, v);
+                    b2 = b1;
+                    b1 = v;
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             // a numerator outside divByRecip's range (zero, whose sign the
-            // corrections would lose, subnormal, huge, Inf) or a row without
-            // a reciprocal: this lane repeats the step with IEEE division
-            if (__builtin_expect(!(nmin >= 0x1p-900 && nmax <= 0x1p900 && recips), 0)) {
+            // corrections would lose, subnormal, Inf) or a row without a
+            // reciprocal: this lane repeats the step with IEEE division
+            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && recips), 0)) {
                 b2 = b2s;
                 b1 = b1s;
                 for (int k = 0; k < SR; k++) {
@@ -455,11 +495,13 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         // the two-operation division q = fma(x, ky, RN(x kz)) = RN(x / k2)
         // (2^-900 <= |x| <= 2^900), kz the low part of 1/k2
         double kz = 0.0;
+        const double ky2 = divRecip2(k2);
+        const bool short2 = ky != 0.0 && k1 != 0.0;
         auto stepK = [&](auto fast, int j, const double (&cur)[SR], double (&ahead)[SR],
                         const __amdgpu_buffer_rsrc_t& out, __amdgpu_buffer_rsrc_t& outAhead) {
             loadStep(ahead, outAhead, j + 2);
             settleStep(cur);
-            double nmin = 0x1p900, nmax = 0x1p-900;
+            double nmin = 0x1p900;
             const double b2s = b2, b1s = b1;
 #pragma unroll
             for (int k = 0; k < SR; k++) {
@@ -467,17 +509,13 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 const double num = t - k1 * b1;
                 double v;
                 if constexpr (decltype(fast)::value) v = __builtin_fma(num, ky, num * kz);
-                else v = divByRecip(num, k2, ky);
+                else v = divByRecip(num, k2, ky2);
                 nmin = __builtin_fmin(nmin, __builtin_fabs(num));
-                if constexpr (!decltype(fast)::value) nmax = __builtin_fmax(nmax, __builtin_fabs(num));
                 store(out, k, v);
                 b2 = b1;
                 b1 = v;
             }
-            // (the two-operation division has no upper limit short of Inf and
-            // NaN, and those stay in the recurrence to the end of the step)
-            if constexpr (decltype(fast)::value) nmax = __builtin_fabs(b1) <= 0x1.fffffffffffffp1023 ? 0.0 : 0x1p1000;
-            if (__builtin_expect(!(nmin >= 0x1p-900 && nmax <= 0x1p900 && ky != 0.0), 0)) {
+            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && short2), 0)) {
                 b2 = b2s;
                 b1 = b1s;
                 for (int k = 0; k < SR; k++) {
@@ -511,6 +549,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             if (j < jc) step(j++, bufA, bufC, rA, rC);
             if (j < jc) step(j++, bufB, bufA, rB, rA);
         }
+        loadTail();  // (not before: the steps that read the ring need the registers)
         auto constSteps = [&](auto fast) {
             int j = jc;
             for (; j + 3 <= nFull; j += 3) {
@@ -522,7 +561,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             if (j < nFull) stepK(fast, j++, bufB, bufA, rB, rA);
         };
         if (jc < nFull) {
-            if (D.fastDiv && k1 != 0.0) {
+            if (D.fastDiv) {
                 kz = __builtin_fma(-k2, ky, 1.0) / k2;
                 constSteps(std::true_type{});
             } else {
@@ -557,10 +596,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
     double a0 = b2 - duEnd * a1;
     at(m - 2) = a0;
     const double xm2 = a0;
-    // the rows left of this sweep, 0 .. rem - 1 (past them, row 0)
     double tailU = du[min(lane, SR - 1)], tailW = dw[min(lane, SR - 1)];
-#pragma unroll
-    for (int k = 0; k < SR; k++) tail[k] = at(max(rem - 1 - k, 0));
     if (nFull > 0) {
         // step j holds rows m-3 - j SR - k; row k of the step sits at offset
         // SR-1-k above the step's lowest row m-3 - j SR - (SR-1)
@@ -594,15 +630,24 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             const int rd = diagRow(j + 1);
             const double p0 = du[rd], p1 = dw[rd];
             loadStep(ahead, outAhead, j + 2);
-            settleStep(cur);
             const int slot = (j - jcb) & 1;
+            RingRows<2> ahead0(sd[slot], 0);
+            settleStep(cur);
 #pragma unroll
-            for (int k = 0; k < SR; k++) {
-                const double t = cur[k] - sd[slot][0][k] * a0;
-                const double v = t - sd[slot][1][k] * a1;
-                store(out, SR - 1 - k, v);
-                a1 = a0;
-                a0 = v;
+            for (int q = 0; q < SR / 4; q++) {
+                RingRows<2> f = ahead0;
+                if (q + 1 < SR / 4) ahead0 = RingRows<2>(sd[slot], 4 * (q + 1));
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int k = 4 * q + i;
+                    const double t = cur[k] - f.v[0][i] * a0;
+                    const double v = t - f.v[1][i] * a1;
+                    store(out, SR - 1 - k, v);
+                    a1 = a0;
+                    a0 = v;
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
             stageDiag(slot ^ 1, p0, p1);
         };
@@ -649,6 +694,9 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         }
     }
     static_assert(SR <= kCHColBlock, "a lane for each row left");
+    // the rows left of this sweep, 0 .. rem - 1 (past them, row 0)
+#pragma unroll
+    for (int k = 0; k < SR; k++) tail[k] = at(max(rem - 1 - k, 0));
 #pragma unroll
     for (int k = 0; k < SR; k++) {
         if (k >= rem) break;
@@ -828,7 +876,7 @@ hipError_t chLaunchRhs(const CHDesc* descs, int count, int totalTiles, int step,
 hipError_t chLaunchTranspose(const CHDesc* descs, int count, int totalTiles, hipStream_t st)
 {
     if (count <= 0 || totalTiles <= 0) return hipSuccess;
-    hipLaunchKernelGGL(chdev::transposeKernel, dim3(totalTiles), dim3(256), 0, st, descs, count);
+    hipLaunchKernelGGL(chdev::transposeKernel, dim3(totalTiles), dim3(chdev::kTrThreads), 0, st, descs, count);
     return hipGetLastError();
 }
 
