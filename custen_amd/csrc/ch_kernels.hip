@@ -276,40 +276,35 @@ __global__ __launch_bounds__(kTrThreads) void transposeKernel(const CHDesc* __re
 // One wave to a CU at 1024 columns: the time is the wave's own instructions,
 // 10 a row forward and 6 backward at about 5 clocks each, of which two export a
 // row at 12, and the latencies that it meets alone; rows outside the constant
-// runs take 16 and 8.  1024 x 1024: 50.4 us, of 57.5 before the loads ahead carried
+// runs take 18 and 8.  1024 x 1024: 50.7 us, of 57.5 before the loads ahead carried
 // over from the one loop to the next, the rows left and the rows of the ends
 // were loaded ahead, the upper limit of the short divisions was found not to
 // need a test in each row, and the ring was read a group ahead (256 x 256, whose
-// factors never settle: 20.9 us, of 25.3; 4096 x 4096: 255, of 290).
+// factors never settle: 22.0 us, of 25.3; 4096 x 4096: 269, of 290).
 // ---------------------------------------------------------------------------
 constexpr int SR = 16;  // rows per step (settleStep takes 16)
 
-// RN(1/d) for the two-operation division when 2^-60 <= |d| <= 2^60, else 0 (the
-// row then divides with IEEE division).
+// Reciprocal of a diagonal entry for the divisions below: RN(1/d) when
+// 2^-60 <= |d| <= 2^60, else 0 (the row then divides with IEEE division).
 __device__ __forceinline__ double divRecip(double d)
 {
     const double ad = __builtin_fabs(d);
     return (ad >= 0x1p-60 && ad <= 0x1p60) ? 1.0 / d : 0.0;
 }
 
-// The GPU's IEEE division (reciprocal estimate, two Newton steps, quotient,
-// remainder, one correction) without its operand scaling and fixup, which leave
-// operands alone in the range below; the reciprocal comes once a row, off the
-// recurrence's critical path, as all columns of a request share the matrix.  The
-// dependent chain is three operations against eleven.  The preconditions (no
-// subnormal intermediate, 2^-60 <= |d| <= 2^60, where divRecip is not 0) hold for
-// |n| >= 2^-900; infinities and NaN need IEEE division.
-__device__ __forceinline__ double divRecip2(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-    const double ad = __builtin_fabs(d);
-    return (ad >= 0x1p-60 && ad <= 0x1p60) ? y : 0.0;
-}
+// n / d, correctly rounded, with y = RN(1/d) precomputed (all columns of a
+// request share the matrix, so y is computed once per row, off the
+// recurrence's critical path).  q0 = RN(n y) and two corrections
+// q <- RN(q + RN(n - d q) y) (each remainder exact by fma) give RN(n / d)
+// (Markstein's theorem: the first correction makes q faithful, the second
+// rounds it correctly); the dependent chain is five operations against the
+// eleven of the scaled IEEE sequence.  The preconditions (no subnormal
+// intermediate) hold for |n| >= 2^-900 and the range of d in divRecip (y != 0);
+// an n so large that q0 overflows makes q NaN.
 __device__ __forceinline__ double divByRecip(double n, double d, double y)
 {
-    const double q = n * y;
+    double q = n * y;
+    q = __builtin_fma(__builtin_fma(-d, q, n), y, q);
     return __builtin_fma(__builtin_fma(-d, q, n), y, q);
 }
 // An infinity or NaN stays in the recurrence to the end of a step, where its
@@ -437,7 +432,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         // row before (uniform)
         bool recips = true;
         auto stageDiag = [&](int slot, double p0, double p1, double p2) {
-            const double y = divRecip2(p2);
+            const double y = divRecip(p2);
             sd[slot][0][lane] = p0;
             sd[slot][1][lane] = p1;
             sd[slot][2][lane] = p2;
@@ -495,7 +490,6 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
         // the two-operation division q = fma(x, ky, RN(x kz)) = RN(x / k2)
         // (2^-900 <= |x| <= 2^900), kz the low part of 1/k2
         double kz = 0.0;
-        const double ky2 = divRecip2(k2);
         const bool short2 = ky != 0.0 && k1 != 0.0;
         auto stepK = [&](auto fast, int j, const double (&cur)[SR], double (&ahead)[SR],
                         const __amdgpu_buffer_rsrc_t& out, __amdgpu_buffer_rsrc_t& outAhead) {
@@ -509,7 +503,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 const double num = t - k1 * b1;
                 double v;
                 if constexpr (decltype(fast)::value) v = __builtin_fma(num, ky, num * kz);
-                else v = divByRecip(num, k2, ky2);
+                else v = divByRecip(num, k2, ky);
                 nmin = __builtin_fmin(nmin, __builtin_fabs(num));
                 store(out, k, v);
                 b2 = b1;
