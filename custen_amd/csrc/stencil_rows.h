@@ -69,7 +69,7 @@ __global__ __launch_bounds__(kLanes) void stencilRows(StencilLaunch a)
     const int bands = rowsBands(bg, 4 * a.chunks);
     const int n = __builtin_amdgcn_readfirstlane((bg.yb - bg.ya + bands - 1) / bands);
     const int yS = min(bg.ya + band * n, bg.yb - n);
-    const int x0 = min(bg.xa + strip * kTW, bg.xb - kTW);
+    const int x0 = bg.x0(strip);
     const int nx = a.nx, L = a.L;
     const Glob<double>* __restrict__ in = globalPtr<double>(a.in);
     Glob<double>* __restrict__ out = globalPtr<double>(a.out);

@@ -103,3 +103,19 @@ def test_batched_grids(gpu, nx, ny):
             f = oracle.apply(f, w, 5, 2, 5, 2, True)
         assert mismatches(o.cpu().numpy(), f) == 0
     b.close()
+
+
+ALIGNED = [("2DXYnp", 5, 2, 5, 2), ("2DXYnp", 3, 0, 3, 2), ("2DXYnp", 3, 2, 3, 1),
+           ("2DXnp", 7, 3, 1, 0), ("2DXnp", 9, 0, 1, 0), ("2DXnp", 9, 8, 1, 0),
+           ("2DXYnp", 9, 4, 9, 4), ("2DXYnp", 7, 0, 7, 6), ("2DYnp", 1, 0, 9, 4)]
+
+
+@pytest.mark.parametrize("variant,H,L,V,T", ALIGNED)
+@pytest.mark.parametrize("nx", [128, 144, 160, 240, 256, 272, 288, 384, 400, 416])
+def test_aligned_rows(gpu, variant, H, L, V, T, nx):
+    """Rows of whole lines: strips at multiples of 128 columns, the first and the
+    last of the window drawn in."""
+    print(f"band window aligned {variant} {H}x{V} L={L} nx={nx}", flush=True)
+    run(gpu, variant, nx, 45, H, L, V, T, (4, 2))
+    run(gpu, variant, nx, 45, H, L, V, T, (4, 8))
+    run(gpu, variant, nx, 45, H, L, V, T, (8, 1), shift=1)
