@@ -32,6 +32,23 @@ struct RowMap {
     int rowMax;
 };
 
+// Source row of region row gy for regions at least as tall as the window: one
+// wrap at most for every row that an output of the region needs.  A tile that
+// runs past the region's end holds rows further on, which no stored output
+// needs; the last row stands in for those that one wrap does not bring back
+// (unlimited, a 32-row tile of a grid of 3 rows would be read 26 rows past the
+// array's end).
+__host__ __device__ inline int mapRowNear(const RowMap& m, int gy)
+{
+    if (m.wrap) {
+        if (gy < 0) return gy + m.rowWrap;
+        if (gy < m.rowWrap) return gy;
+        gy -= m.rowWrap;
+        return gy < m.rowWrap ? gy : m.rowWrap - 1;
+    }
+    return gy < m.rowMin ? m.rowMin : (gy > m.rowMax ? m.rowMax : gy);
+}
+
 // One stencil apply over a rectangular region of rows [0, ny) of a grid that
 // is nx wide.  Output row gy is written at out + gy * ldOut.
 struct StencilLaunch {

@@ -177,21 +177,10 @@ struct StagedRows {
     T halo[2];
 };
 
-// Source row of region row gy when the region is at least as tall as the
-// window (one correction at most); the general mapRow otherwise.
-__device__ __forceinline__ int mapRowNear(const RowMap& m, int gy)
-{
-    if (m.wrap) {
-        if (gy < 0) gy += m.rowWrap;
-        else if (gy >= m.rowWrap) gy -= m.rowWrap;
-        return gy;
-    }
-    return gy < m.rowMin ? m.rowMin : (gy > m.rowMax ? m.rowMax : gy);
-}
-
-// FAST: the strip is a full 128 columns of pair-aligned rows, and row and
-// halo-column indices need at most one wrap (ny >= window height, nx >= 128
-// > any extent): no division in the address arithmetic.
+// FAST: the strip is a full 128 columns of pair-aligned rows, and the rows that
+// stored outputs need and halo columns take one wrap at most (ny >= window
+// height, nx >= 128 > any extent): no division in the address arithmetic
+// (mapRowNear).
 template <typename T, int NR, bool FAST, int CPL = 2>
 __device__ __forceinline__ void loadRows(StagedRows<T, NR, CPL>& s, const Glob<T>* __restrict__ in,
                                          int64_t ldIn, const RowMap& rows, int y0, int T_, int x0,
