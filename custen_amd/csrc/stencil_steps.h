@@ -73,6 +73,16 @@ __host__ __device__ inline bool stepsApply(int nx, int ny)
     return nx >= kTW && nx < (1 << 28) && ny >= 16;
 }
 
+// Rows that lanes wrote to LDS may be read by other lanes of the wave from here
+// on.  The LDS takes a wave's operations in order, so this costs no
+// instruction, but the compiler sees one lane, whose reads of its neighbours'
+// columns do not alias what it wrote, and might move them up.
+__device__ __forceinline__ void rowsWritten()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // K steps of wave item g of a grid (periodic, nx x ny, row stride nx).  `lds`
 // is the wave's StepsShape::ELEMS elements.
 template <typename T, int H, int V, int K>
@@ -221,6 +231,7 @@ __device__ __forceinline__ void stepsWalk(const Glob<T>* __restrict__ in, Glob<T
             if (t >= k * V) addRow(acc[k], v[k], pc);
             __builtin_amdgcn_sched_barrier(0);
         }
+        rowsWritten();
         const int o = t - (V - 1) - (K - 1) * V;
         if (o >= 0 && o < n) {
             const V2 r = {acc[K - 1][done][0], acc[K - 1][done][1]};
