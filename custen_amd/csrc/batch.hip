@@ -52,9 +52,10 @@ namespace dev {
 
 // The single-grid launch description of grid G (periodic xy, all points
 // written), reading the side given by the step parity.
-__device__ __forceinline__ StencilLaunch gridLaunch(const BatchDev& G, int parity, Dtype dt,
-                                                    const double* weights, int H, int L, int V,
-                                                    int Tt, int rpw, int chunks)
+__host__ __device__ __forceinline__ StencilLaunch gridLaunch(const BatchDev& G, int parity,
+                                                             Dtype dt, const double* weights,
+                                                             int H, int L, int V, int Tt, int rpw,
+                                                             int chunks)
 {
     StencilLaunch a;
     a.dtype = dt;
@@ -315,12 +316,9 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
     for (int k = 0; k < kItemKinds; k++) items[k].assign(b->numGrids, 0);
     for (int i = 0; i < b->numGrids; i++) {
         BatchDev& d = b->host[i];
-        StencilLaunch one{};
-        one.ny = one.wy1 = one.rows.rowWrap = d.ny;
-        one.wx1 = d.nx;
-        one.V = b->V;
-        one.rows.wrap = 1;
-        one.chunks = chunks;
+        // (what the kernels make of the grid, so that both count the same items)
+        const StencilLaunch one = dev::gridLaunch(d, 0, b->dtype, b->dWeights, b->H, b->L, b->V,
+                                                  b->T, rpw, chunks);
         d.walked = band && dev::bandApplies(one, rpw) ? 1 : 0;
         d.stepped = passes && dev::stepsApply(d.nx, d.ny) ? 1 : 0;
         d.stripBase = (int)n[kAllStrips];

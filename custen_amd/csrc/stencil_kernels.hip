@@ -422,8 +422,9 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
         if (s.band && dev::bandApplies(s, RPW)) {
             const dev::BandGrid g = dev::bandGrid(s, RPW);
             if constexpr (dev::kStreamRows<T, H, V>) {
+                static_assert(RPW == dev::kRowsRPW, "stencilRows counts bands in chunks of 4 rows");
                 if (s.chunks * RPW >= dev::kStreamBand) {
-                    const int64_t rowWaves = (int64_t)g.strips * dev::rowsBands(g, s.chunks * RPW);
+                    const int64_t rowWaves = (int64_t)g.strips * dev::rowsBands(g, s.chunks);
                     if (rowWaves > 0x7fffffff) return hipErrorInvalidValue;
                     hipLaunchKernelGGL((dev::stencilRows<H, V>), dim3((unsigned)rowWaves),
                                        dim3(dev::kLanes), 0, st, s);

@@ -37,9 +37,12 @@ struct RowsShape {
     static constexpr int NS = 34;                      // weights in scalar registers
 };
 
-// Bands of about `most` rows, of equal length; the last ends at the last row.
-__host__ __device__ inline int rowsBands(const BandGrid& g, int most)
+// Bands of about 4 * chunks rows, of equal length; the last ends at the last
+// row.  (The host counts waves with the same function.)
+constexpr int kRowsRPW = 4;
+__host__ __device__ inline int rowsBands(const BandGrid& g, int chunks)
 {
+    const int most = kRowsRPW * chunks;
     return (g.yb - g.ya + most - 1) / most;
 }
 
@@ -63,10 +66,10 @@ __global__ __launch_bounds__(kLanes) void stencilRows(StencilLaunch a)
     }
 
     const int lane = threadIdx.x;
-    const BandGrid bg = bandGrid(a, 4);
+    const BandGrid bg = bandGrid(a, kRowsRPW);
     const int g = xcdRemap(blockIdx.x, gridDim.x);
     const int strip = g % bg.strips, band = g / bg.strips;
-    const int bands = rowsBands(bg, 4 * a.chunks);
+    const int bands = rowsBands(bg, a.chunks);
     const int n = __builtin_amdgcn_readfirstlane((bg.yb - bg.ya + bands - 1) / bands);
     const int yS = min(bg.ya + band * n, bg.yb - n);
     const int x0 = bg.x0(strip);
