@@ -102,16 +102,22 @@ struct FunLaunch {
     int band;                // as StencilLaunch::band (weighted-sum built-ins)
 };
 
-hipError_t launchStencil(const StencilLaunch& s, hipStream_t stream);
-hipError_t launchFun(const FunLaunch& f, hipStream_t stream);
+// What a launch runs (custenGetBandMode, mem_shared).
+struct KernelUse {
+    int band = 0;      // the band walker, its row-streaming form included
+    int ldsBytes = 0;  // of a workgroup
+};
+
+// With `use`, nothing is launched: it is set to what would be (launchFun leaves
+// it alone for functions that do not run on the stencil kernels).
+hipError_t launchStencil(const StencilLaunch& s, hipStream_t stream, KernelUse* use = nullptr);
+hipError_t launchFun(const FunLaunch& f, hipStream_t stream, KernelUse* use = nullptr);
 
 // Device addresses of the built-in point functions on the current device.
 hipError_t builtinFunctionAddress(Builtin b, void** addr);
 
-// LDS bytes the stencil kernel uses for a given shape (reported in mem_shared).
+// LDS bytes of a strip-kernel workgroup.
 int stencilLdsBytes(Dtype dt, int H, int V, int rowsPerWave);
-// LDS bytes of one band-walker workgroup (one wave).
-int stencilBandLdsBytes(Dtype dt, int H, int V, int rowsPerWave);
 // chunks per band (4 rows each) with which a shape that can streams its rows; 0: none
 int stencilRowsChunks(Dtype dt, int H, int V, int nx, int ny);
 

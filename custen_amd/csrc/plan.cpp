@@ -260,6 +260,8 @@ Builtin recognise(const double* func, int device)
     return found;
 }
 
+KernelUse kernelUse(const cuSten_t* h, const Plan* p);
+
 void createCommon(cuSten_t* h, const CreateArgs& a)
 {
     if (h == nullptr) {
@@ -317,7 +319,6 @@ void createCommon(cuSten_t* h, const CreateArgs& a)
     h->yGrid = (h->nyTile + a.BY - 1) / a.BY;
     h->nxLocal = (a.dir == Dir::Y) ? a.BX : a.BX + a.L + a.R;
     h->nyLocal = (a.dir == Dir::X) ? a.BY : a.BY + a.T + a.B;
-    h->mem_shared = a.weno ? wenoLdsBytes(0) : stencilLdsBytes(a.dtype, p->H, p->V, 0);
     if (a.weno) {
         // custenCreateDestroy2DXYADVWENOp.cu:99-117: coefficients 1/dx, 1/dy,
         // a 7 x 7 window (3 points each side)
@@ -382,6 +383,7 @@ void createCommon(cuSten_t* h, const CreateArgs& a)
         h->numBoundaryBottom = a.B * a.nx;
         setBoundaries(h, p, a.in, !a.periodic && a.dir == Dir::Y);
     }
+    h->mem_shared = kernelUse(h, p).ldsBytes;
 }
 
 // ---------------------------------------------------------------------------
@@ -425,8 +427,9 @@ struct Region {
     const double* v = nullptr;
 };
 
+// With `use`, what would be launched (KernelUse) instead of launching it.
 hipError_t launchRegion(const cuSten_t* h, const Plan* p, const Region& r, const double* params,
-                        hipStream_t st)
+                        hipStream_t st, KernelUse* use = nullptr)
 {
     const int R = p->H - 1 - p->L;
     const int B = p->V - 1 - p->T;
@@ -434,6 +437,7 @@ hipError_t launchRegion(const cuSten_t* h, const Plan* p, const Region& r, const
     const int wx1 = p->periodic ? h->nx : h->nx - R;
     const int wy0 = p->periodic ? 0 : p->T;
     const int wy1 = p->periodic ? h->ny : h->ny - B;
+    if (use && (p->weno || p->pointLauncher)) return hipSuccess;
     if (p->weno) {
         WenoLaunch w{};
         w.in = static_cast<const double*>(r.in);
@@ -487,7 +491,7 @@ hipError_t launchRegion(const cuSten_t* h, const Plan* p, const Region& r, const
             const bool user = p->rowsPerWave || p->chunks || p->colsPerLane;
             s.band = !user && p->tuned && p->tunedBand ? 1 : 0;
         }
-        return launchStencil(s, st);
+        return launchStencil(s, st, use);
     }
     if (p->pointLauncher) {
         // the caller's kernel with its point function inlined (custen_point.h)
@@ -551,7 +555,39 @@ hipError_t launchRegion(const cuSten_t* h, const Plan* p, const Region& r, const
         const bool user = p->rowsPerWave || p->chunks || p->colsPerLane;
         f.band = !user && p->tuned && p->tunedBand ? 1 : 0;
     }
-    return launchFun(f, st);
+    return launchFun(f, st, use);
+}
+
+// The whole grid, resident on the device.
+Region residentRegion(const cuSten_t* h, const Plan* p)
+{
+    Region r;
+    r.in = h->dataInput[0];
+    r.out = h->dataOutput[0];
+    r.ldIn = h->nx;
+    r.ldOut = h->nx;
+    r.nx = h->nx;
+    r.ny = h->ny;
+    r.rows.wrap = p->periodic ? 1 : 0;
+    r.rows.rowWrap = p->periodic ? h->ny : 0;
+    r.rows.rowMin = 0;
+    r.rows.rowMax = h->ny - 1;
+    r.yGlobal0 = 0;
+    if (p->weno) {
+        r.u = h->uVel[0];
+        r.v = h->vVel[0];
+    }
+    return r;
+}
+
+// What Compute runs on the resident grid with the configuration in force.
+KernelUse kernelUse(const cuSten_t* h, const Plan* p)
+{
+    KernelUse u;
+    u.ldsBytes = p->weno ? wenoLdsBytes(p->rowsPerWave)
+                         : stencilLdsBytes(p->dtype, p->H, p->V, p->rowsPerWave);
+    (void)launchRegion(h, p, residentRegion(h, p), nullptr, nullptr, &u);
+    return u;
 }
 
 bool tablesConsistent(const cuSten_t* h, const Plan* p)
@@ -762,29 +798,7 @@ void computeCommon(cuSten_t* h, bool offload, const char* fn)
                                         resident ? st : h->streams[1], fn);
     if (src != nullptr && count > 0 && params == nullptr) return;
     if (resident) {
-        Region r;
-        r.in = in;
-        r.out = out;
-        r.ldIn = h->nx;
-        r.ldOut = h->nx;
-        r.nx = h->nx;
-        r.ny = h->ny;
-        if (p->periodic) {
-            r.rows.wrap = 1;
-            r.rows.rowWrap = h->ny;
-            r.rows.rowMin = 0;
-            r.rows.rowMax = h->ny - 1;
-        } else {
-            r.rows.wrap = 0;
-            r.rows.rowWrap = 0;
-            r.rows.rowMin = 0;
-            r.rows.rowMax = h->ny - 1;
-        }
-        r.yGlobal0 = 0;
-        if (p->weno) {
-            r.u = h->uVel[0];
-            r.v = h->vVel[0];
-        }
+        const Region r = residentRegion(h, p);
         // First resident Compute of a large grid: pick the tile configuration
         // (bit-identical results for every candidate; synchronous once).
         if (!p->weno && !p->tuned && !p->band && p->rowsPerWave == 0 && p->chunks == 0 &&
@@ -841,6 +855,7 @@ void computeCommon(cuSten_t* h, bool offload, const char* fn)
             p->tunedChunks = v.chunks;
             p->tunedCpl = v.cpl;
             p->tunedBand = v.band != 0;
+            h->mem_shared = kernelUse(h, p).ldsBytes;
         }
         e = launchRegion(h, p, r, params, st);
         if (e != hipSuccess) setHipError(e, fn);
@@ -1224,7 +1239,7 @@ void custenSetTileConfigEx(cuSten_t* h, int rowsPerWave, int chunksPerGroup, int
     p->band = false;
     if (rowsPerWave == 0 && chunksPerGroup == 0 && columnsPerLane == 0)
         p->tuned = false;  // re-tune on next Compute
-    h->mem_shared = stencilLdsBytes(p->dtype, p->H, p->V, rowsPerWave);
+    h->mem_shared = kernelUse(h, p).ldsBytes;
 }
 
 void custenSetBandConfig(cuSten_t* h, int rowsPerWave, int chunksPerBand)
@@ -1243,7 +1258,7 @@ void custenSetBandConfig(cuSten_t* h, int rowsPerWave, int chunksPerBand)
     p->chunks = chunksPerBand;
     p->colsPerLane = 2;
     p->band = true;
-    h->mem_shared = stencilBandLdsBytes(p->dtype, p->H, p->V, rowsPerWave);
+    h->mem_shared = kernelUse(h, p).ldsBytes;
 }
 
 int custenGetBandMode(cuSten_t* h)
@@ -1251,7 +1266,8 @@ int custenGetBandMode(cuSten_t* h)
     Plan* p = planOf(h, "custenGetBandMode");
     if (!p) return -CUSTEN_ERROR_INVALID_VALUE;
     const bool user = p->rowsPerWave || p->chunks || p->colsPerLane;
-    return (p->band || (!user && p->tuned && p->tunedBand)) ? 1 : 0;
+    if (user || p->tuned) return (p->band || (!user && p->tunedBand)) ? 1 : 0;
+    return kernelUse(h, p).band;
 }
 
 void custenSetTileConfig(cuSten_t* h, int rowsPerWave, int chunksPerGroup)

@@ -410,7 +410,7 @@ int gridSize(int nx, int ny, int TH, int chunks)
 // interior strip at all: unaligned rows, or a periodic grid lower than the
 // stencil) as the contiguous ranges left and right of the interior.
 template <typename T, int H, int V, int RPW, Xform X, int CPL = 2>
-hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
+hipError_t runFixed(const StencilLaunch& in, hipStream_t st, KernelUse* use)
 {
     StencilLaunch s = in;
     // band walker: every weight stencil shape, and the cube-minus point
@@ -424,12 +424,20 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
             if constexpr (dev::kStreamRows<T, H, V>) {
                 static_assert(RPW == dev::kRowsRPW, "stencilRows counts bands in chunks of 4 rows");
                 if (s.chunks * RPW >= dev::kStreamBand) {
+                    if (use) {
+                        *use = {1, dev::RowsShape<H, V>::LDS_BYTES};
+                        return hipSuccess;
+                    }
                     const int64_t rowWaves = (int64_t)g.strips * dev::rowsBands(g, s.chunks);
                     if (rowWaves > 0x7fffffff) return hipErrorInvalidValue;
                     hipLaunchKernelGGL((dev::stencilRows<H, V>), dim3((unsigned)rowWaves),
                                        dim3(dev::kLanes), 0, st, s);
                     return hipGetLastError();
                 }
+            }
+            if (use) {
+                *use = {1, dev::BandShape<T, H, V, RPW>::LDS_BYTES};
+                return hipSuccess;
             }
             const int64_t waves = (int64_t)g.strips * g.bands;
             if (waves > 0x7fffffff) return hipErrorInvalidValue;
@@ -439,6 +447,10 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
         }
     }
     const int tw = dev::kLanes * CPL;
+    if (use) {
+        *use = {0, (int)sizeof(T) * (dev::kWaves * RPW + V - 1) * dev::ldsRowLengthW(tw, H)};
+        return hipSuccess;
+    }
     const int tilesX = (s.nx + tw - 1) / tw;
     const int rowsPerGroup = dev::kWaves * RPW * s.chunks;
     const int tilesY = (s.ny + rowsPerGroup - 1) / rowsPerGroup;
@@ -492,13 +504,17 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st)
 }
 
 template <typename T, Xform X>
-hipError_t runGeneric(const StencilLaunch& s, hipStream_t st)
+hipError_t runGeneric(const StencilLaunch& s, hipStream_t st, KernelUse* use)
 {
     const int TH = dev::kWaves * dev::kGenericRPW;
     const int grid = gridSize(s.nx, s.ny, TH, s.chunks);
     const size_t lds =
         sizeof(T) * ((size_t)(TH + s.V - 1) * dev::ldsRowLength(s.H) + (size_t)s.H * s.V);
     if (lds > 160 * 1024) return hipErrorInvalidValue;
+    if (use) {
+        *use = {0, (int)lds};
+        return hipSuccess;
+    }
     if (lds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&dev::stencilGeneric<T, X>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -518,31 +534,31 @@ hipError_t runGeneric(const StencilLaunch& s, hipStream_t st)
     X_(11, 1) X_(13, 1) X_(1, 11) X_(1, 13) X_(7, 7) X_(9, 9) X_(3, 5) X_(5, 3)
 
 template <typename T, Xform X>
-hipError_t dispatchTyped(const StencilLaunch& s, hipStream_t st)
+hipError_t dispatchTyped(const StencilLaunch& s, hipStream_t st, KernelUse* use)
 {
     const int rpw = s.rowsPerWave;
     // one column per lane (deeper row blocking) for the xy shapes
     if (s.colsPerLane == 1) {
         if (s.H == 5 && s.V == 5)
-            return rpw == 16 ? runFixed<T, 5, 5, 16, X, 1>(s, st) : runFixed<T, 5, 5, 8, X, 1>(s, st);
+            return rpw == 16 ? runFixed<T, 5, 5, 16, X, 1>(s, st, use) : runFixed<T, 5, 5, 8, X, 1>(s, st, use);
         if (s.H == 3 && s.V == 3)
-            return rpw == 16 ? runFixed<T, 3, 3, 16, X, 1>(s, st) : runFixed<T, 3, 3, 8, X, 1>(s, st);
+            return rpw == 16 ? runFixed<T, 3, 3, 16, X, 1>(s, st, use) : runFixed<T, 3, 3, 8, X, 1>(s, st, use);
     }
 #define CUSTEN_CASE(HH, VV)                                                      \
     if (s.H == HH && s.V == VV) {                                                \
-        if (rpw == 4) return runFixed<T, HH, VV, 4, X>(s, st);                   \
-        return runFixed<T, HH, VV, 8, X>(s, st);                                 \
+        if (rpw == 4) return runFixed<T, HH, VV, 4, X>(s, st, use);                   \
+        return runFixed<T, HH, VV, 8, X>(s, st, use);                                 \
     }
     CUSTEN_FIXED_SHAPES(CUSTEN_CASE)
 #undef CUSTEN_CASE
     // wider shapes (high-order schemes), identity transform, 4 rows per wave
     if constexpr (X == Xform::Identity) {
 #define CUSTEN_WIDE(HH, VV) \
-    if (s.H == HH && s.V == VV) return runFixed<T, HH, VV, 4, X>(s, st);
+    if (s.H == HH && s.V == VV) return runFixed<T, HH, VV, 4, X>(s, st, use);
         CUSTEN_WIDE_SHAPES(CUSTEN_WIDE)
 #undef CUSTEN_WIDE
     }
-    return runGeneric<T, X>(s, st);
+    return runGeneric<T, X>(s, st, use);
 }
 
 }  // namespace
@@ -583,15 +599,7 @@ int stencilRowsChunks(Dtype dt, int H, int V, int nx, int ny)
     return best;
 }
 
-int stencilBandLdsBytes(Dtype dt, int H, int V, int rowsPerWave)
-{
-    const int rpw = rowsPerWave == 8 ? 8 : 4;
-    const int d = 8 / rpw;
-    const int hlp = H & ~1;  // H - 1 halo columns per side, rounded up to even
-    return (dt == Dtype::F64 ? 8 : 4) * ((d + 1) * rpw + V - 1) * (dev::kTW + 2 * hlp);
-}
-
-hipError_t launchStencil(const StencilLaunch& in, hipStream_t st)
+hipError_t launchStencil(const StencilLaunch& in, hipStream_t st, KernelUse* use)
 {
     StencilLaunch s = in;
     if (s.nx <= 0 || s.ny <= 0) return hipSuccess;
@@ -617,16 +625,16 @@ hipError_t launchStencil(const StencilLaunch& in, hipStream_t st)
     if (s.dtype == Dtype::F64) {
         s.vecIn = pairAligned<double>(s.in, s.ldIn);
         s.vecOut = pairAligned<double>(s.out, s.ldOut);
-        if (s.xform == Xform::CubeMinus) return dispatchTyped<double, Xform::CubeMinus>(s, st);
-        return dispatchTyped<double, Xform::Identity>(s, st);
+        if (s.xform == Xform::CubeMinus) return dispatchTyped<double, Xform::CubeMinus>(s, st, use);
+        return dispatchTyped<double, Xform::Identity>(s, st, use);
     }
     s.vecIn = pairAligned<float>(s.in, s.ldIn);
     s.vecOut = pairAligned<float>(s.out, s.ldOut);
     if (s.xform == Xform::CubeMinus) return hipErrorInvalidValue;
-    return dispatchTyped<float, Xform::Identity>(s, st);
+    return dispatchTyped<float, Xform::Identity>(s, st, use);
 }
 
-hipError_t launchFun(const FunLaunch& in, hipStream_t st)
+hipError_t launchFun(const FunLaunch& in, hipStream_t st, KernelUse* use)
 {
     FunLaunch f = in;
     if (f.nx <= 0 || f.ny <= 0) return hipSuccess;
@@ -664,8 +672,9 @@ hipError_t launchFun(const FunLaunch& in, hipStream_t st)
         s.chunks = f.chunks;
         s.colsPerLane = f.colsPerLane;
         s.band = f.band;
-        return launchStencil(s, st);
+        return launchStencil(s, st, use);
     }
+    if (use) return hipSuccess;
     if (f.chunks <= 0) f.chunks = kDefaultChunks;
 
     const int TH = dev::kWaves * dev::kFunRPW;

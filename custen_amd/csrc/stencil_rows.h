@@ -35,6 +35,7 @@ struct RowsShape {
     static constexpr int HLP = ((H - 1) + 1) & ~1;     // halo columns staged per side
     static constexpr int LD = kTW + 2 * HLP;
     static constexpr int NS = 34;                      // weights in scalar registers
+    static constexpr int LDS_BYTES = D * LD * 8;
 };
 
 // Bands of about 4 * chunks rows, of equal length; the last ends at the last

@@ -300,8 +300,10 @@ void custenSetStream(cuSten_t* pt_cuSten, hipStream_t stream);
 void custenSetTileConfig(cuSten_t* pt_cuSten, int rowsPerWave, int chunksPerGroup);
 void custenSetTileConfigEx(cuSten_t* pt_cuSten, int rowsPerWave, int chunksPerGroup,
                            int columnsPerLane);
-/* The configuration Compute uses: the caller's, else the autotuner's (all 0
- * before the first tuned Compute). */
+/* The configuration Compute uses: the caller's, else the autotuner's.  All 0:
+ * the default, which is the band walker on every grid that it covers (see
+ * custenGetBandMode), before the first tuned Compute and for grids that are
+ * not tuned (under 2^20 points, host-resident, or captured first). */
 int custenGetTileConfig(cuSten_t* pt_cuSten, int* rowsPerWave, int* chunksPerGroup,
                         int* columnsPerLane);
 
@@ -316,8 +318,9 @@ int custenGetTileConfig(cuSten_t* pt_cuSten, int* rowsPerWave, int* chunksPerGro
  * kernel with the same rowsPerWave and chunks.  custenSetTileConfig[Ex]
  * switches it off again. */
 void custenSetBandConfig(cuSten_t* pt_cuSten, int rowsPerWave, int chunksPerBand);
-/* 1 if Compute uses the band walker (set by the caller or chosen by the
- * autotuner), 0 if not, negative on error. */
+/* 1 if Compute uses the band walker (set by the caller, chosen by the
+ * autotuner, or by default on a grid that it covers), 0 if not, negative on
+ * error. */
 int custenGetBandMode(cuSten_t* pt_cuSten);
 
 /* WENO handles: 1 (default) squares the smoothness terms in single precision
