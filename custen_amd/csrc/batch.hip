@@ -19,6 +19,7 @@
 
 #include "../../include/cuSten.h"
 #include "../../include/custen_batch.h"
+#include "batch_rules.h"
 #include "kernels.h"
 #include "plan_internal.h"
 #include "stencil_band.h"
@@ -191,6 +192,7 @@ struct custenBatch {
     double* dWeights = nullptr;
     int parity = 0;           // 1: the current input is the original output side
     bool tuned = false;
+    bool configured = false;  // by the caller: every step a launch of its own
     hipStream_t own = nullptr;
     std::map<std::pair<int, int>, hipGraphExec_t> graphs;  // (steps, start parity)
     std::map<std::pair<int, int>, hipGraph_t> graphDefs;
@@ -251,66 +253,22 @@ hipError_t launchAll(const custenBatch* b, ItemKind kind, int parity, hipStream_
     return launchItems(b, 0, b->total[kind], parity, st, kind);
 }
 
-// Several steps in one pass pay once the two sides no longer stay in the L2s
-// (8 x 4 MiB): single steps then wait for memory, and a pass takes a third of
-// its traffic.  In L2 a single step costs 4-6 us and a pass is bound by its
-// chain of rows.  31 steps, single against passes, in us, by MiB a side:
-//   FP64 5x5   16: 196, 288   32:  470, 412   64:  957, 699   128: 1720, 1164
-//   FP32 5x5   16: 220, 280   32:  560, 429   64: 1056, 707
-//   FP64 3x3   16: 174, 160   32:  495, 238   64:  918, 434   128: 1668, 760
-//   FP32 3x3   16: 188, 165   32:  516, 279   64:  979, 552
-constexpr int64_t kStepBytes5 = 24 << 20, kStepBytes3 = 16 << 20;
-// Most rows of a pass's band.  Short bands repeat more rows (V - 1 for each
-// step) and long ones come in few rounds of waves.  In FP64 a batch takes the
-// length of 128, 64, 32, 16 for which rounds times rows is least, where a wave
-// holds 11 KB of LDS (14 on a CU) and the last round counts 0.4.  In FP32, with
-// twice as many waves on a CU, it takes the longest that gives 12 waves to a
-// CU.  5x5, us per step, by rows:
-//   FP64, forty 2048 x 2048 grids     64: 268   128: 262   256: 268
-//   FP64, sixteen 2048 x 2048 grids   64: 115   128: 125
-//   FP64, sixteen 1024 x 1024 grids   16: 41.3   32: 37.5
-//   FP32, sixteen 2048 x 2048 grids   64: 69.5   128: 64.1
-//   FP32, 32 1024 x 1024 grids        32: 43.8   64: 37.5
-constexpr int kStepRows = 128;
-constexpr int kStepSlots = 14 * 256, kStepWaves32 = 12 * 256;
-
 // Item tables for a tile configuration (host copy and device copy): all
 // strips (per-grid loop and strip-only steps); with the band walker, its
 // items for the grids it applies to (at least a strip wide and a chunk and
-// the stencil high) and the strips of the others; and, for a batch that
-// outgrows the L2s, the same for passes of several steps.
+// the stencil high) and the strips of the others; and the same for passes of
+// several steps (batch_rules.h).
 hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
 {
     b->rpw = rpw;
     b->chunks = chunks;
     b->band = band;
-    auto stepItems = [&](const BatchDev& d, int n) -> int64_t {
-        const dev::StepsGrid g =
-            b->dtype == Dtype::F64
-                ? (b->H == 5 ? dev::stepsGrid<double, 5>(d.nx, d.ny, n)
-                             : dev::stepsGrid<double, 3>(d.nx, d.ny, n))
-                : (b->H == 5 ? dev::stepsGrid<float, 5>(d.nx, d.ny, n)
-                             : dev::stepsGrid<float, 3>(d.nx, d.ny, n));
-        return (int64_t)g.strips * g.bands;
-    };
-    int64_t stepBytes = 0;
-    for (const BatchDev& d : b->host)
-        if (dev::stepsApply(d.nx, d.ny))
-            stepBytes += (int64_t)d.nx * d.ny * (b->dtype == Dtype::F64 ? 8 : 4);
-    const bool passes = stepBytes > (b->H == 5 ? kStepBytes5 : kStepBytes3);
-    double least = 0;
-    for (int rows = kStepRows; rows >= 16; rows /= 2) {
-        int64_t waves = 0;
-        for (const BatchDev& d : b->host)
-            if (dev::stepsApply(d.nx, d.ny)) waves += stepItems(d, rows);
-        const double time = std::max(1.0, (double)waves / kStepSlots + 0.4) *
-                            (rows + dev::kFusedSteps * (b->V - 1) + 6);
-        if (rows == kStepRows || b->dtype == Dtype::F32 || time < least) {
-            least = time;
-            b->stepRows = rows;
-        }
-        if (b->dtype == Dtype::F32 && waves >= kStepWaves32) break;
-    }
+    const int size = b->dtype == Dtype::F64 ? 8 : 4;
+    std::vector<GridSize> sizes;
+    for (const BatchDev& d : b->host) sizes.push_back({d.nx, d.ny});
+    const StepsChoice steps = chooseSteps(sizes, size, b->H, b->configured);
+    b->stepRows = steps.rows;
+    const bool passes = std::count(steps.stepped.begin(), steps.stepped.end(), 1) > 0;
     int64_t n[kItemKinds] = {};
     std::vector<int64_t> items[kItemKinds];  // of each grid
     for (int k = 0; k < kItemKinds; k++) items[k].assign(b->numGrids, 0);
@@ -320,7 +278,7 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
         const StencilLaunch one = dev::gridLaunch(d, 0, b->dtype, b->dWeights, b->H, b->L, b->V,
                                                   b->T, rpw, chunks);
         d.walked = band && dev::bandApplies(one, rpw) ? 1 : 0;
-        d.stepped = passes && dev::stepsApply(d.nx, d.ny) ? 1 : 0;
+        d.stepped = steps.stepped[i];
         d.stripBase = (int)n[kAllStrips];
         d.restBase = (int)n[kRestStrips];
         d.bandBase = (int)n[kBands];
@@ -335,8 +293,12 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
         } else if (band) {
             items[kRestStrips][i] = strips;
         }
-        if (d.stepped) items[kSteps][i] = stepItems(d, b->stepRows);
-        else if (passes) items[kStepsRest][i] = strips;
+        if (d.stepped) {
+            const dev::StepsGrid g = dev::stepsGrid(size, b->H, d.nx, d.ny, steps.rows);
+            items[kSteps][i] = (int64_t)g.strips * g.bands;
+        } else if (passes) {
+            items[kStepsRest][i] = strips;
+        }
         for (int k = 0; k < kItemKinds; k++) {
             n[k] += items[k][i];
             if (n[k] > (int64_t)0x7fffffff) return hipErrorInvalidValue;
@@ -593,6 +555,7 @@ extern "C" int custenBatchSetTileConfig(custenBatch* b, int rowsPerWave, int chu
         for (auto& kv : b->graphDefs) (void)hipGraphDestroy(kv.second);
         b->graphs.clear();
         b->graphDefs.clear();
+        b->configured = true;
         e = configure(b, rowsPerWave, chunks, band != 0);
     }
     if (e != hipSuccess) {

@@ -1,0 +1,111 @@
+// batch_rules.h -- which grids of a batch take several steps in one pass over
+// memory (stencil_steps.h), and in bands of how many rows.
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <vector>
+
+namespace custen {
+namespace dev {
+
+constexpr int kFusedSteps = 3;
+
+// Columns that a strip of a pass of K steps stores, of 128: whole 64-byte pieces
+// (with 124 and 120 FP32 columns the pass was 10-15 % slower for the lines
+// shared by two strips).
+__host__ __device__ constexpr int stepsColumns(int size, int H, int K)
+{
+    return (128 - (K - 1) * (H - 1)) / (64 / size) * (64 / size);
+}
+
+// Strips and bands of a grid's pass: bands of `rows` rows, at most `most`.
+struct StepsGrid {
+    int strips, bands, rows;
+};
+__host__ __device__ inline StepsGrid stepsGrid(int size, int H, int nx, int ny, int most)
+{
+    StepsGrid g;
+    const int ow = stepsColumns(size, H, kFusedSteps);
+    g.strips = (nx + ow - 1) / ow;
+    g.bands = (ny + most - 1) / most;
+    g.rows = (ny + g.bands - 1) / g.bands;
+    return g;
+}
+
+// One wrap correction must do for every column and row a wave starts at, and a
+// row's bytes for the 31 bits of a buffer's range.
+inline bool stepsApply(int nx, int ny) { return nx >= 128 && nx < (1 << 28) && ny >= 16; }
+
+}  // namespace dev
+
+// Several steps in one pass pay once the two sides no longer stay in the L2s
+// (8 x 4 MiB): single steps then wait for memory, and a pass takes a third of
+// its traffic.  In L2 a single step costs 4-6 us and a pass is bound by its
+// chain of rows.  31 steps, single against passes, in us, by MiB a side:
+//   FP64 5x5   16: 196, 288   32:  470, 412   64:  957, 699   128: 1720, 1164
+//   FP32 5x5   16: 220, 280   32:  560, 429   64: 1056, 707
+//   FP64 3x3   16: 174, 160   32:  495, 238   64:  918, 434   128: 1668, 760
+//   FP32 3x3   16: 188, 165   32:  516, 279   64:  979, 552
+constexpr int64_t kStepBytes5 = 24 << 20, kStepBytes3 = 16 << 20;
+// Most rows of a pass's band.  Short bands repeat more rows (V - 1 for each
+// step) and long ones come in few rounds of waves.  In FP64 a batch takes the
+// length of 128, 64, 32, 16 for which rounds times rows is least, where a wave
+// holds 11 KB of LDS (14 on a CU) and the last round counts 0.4.  In FP32, with
+// twice as many waves on a CU, it takes the longest that gives 12 waves to a
+// CU.  5x5, us per step, by rows:
+//   FP64, forty 2048 x 2048 grids     64: 268   128: 262   256: 268
+//   FP64, sixteen 2048 x 2048 grids   64: 115   128: 125
+//   FP64, sixteen 1024 x 1024 grids   16: 41.3   32: 37.5
+//   FP32, sixteen 2048 x 2048 grids   64: 69.5   128: 64.1
+//   FP32, 32 1024 x 1024 grids        32: 43.8   64: 37.5
+constexpr int kStepRows = 128;
+constexpr int kStepSlots = 14 * 256, kStepWaves32 = 12 * 256;
+
+struct GridSize {
+    int nx, ny;
+};
+struct StepsChoice {
+    std::vector<char> stepped;  // of each grid
+    int rows = 16;              // most rows per band
+};
+
+// What a batch of H x H stencils on elements of `size` bytes takes in passes.
+// `single`: the caller configured single steps.
+inline StepsChoice chooseSteps(const std::vector<GridSize>& grids, int size, int H, bool single)
+{
+    StepsChoice c;
+    c.stepped.assign(grids.size(), 0);
+    int64_t bytes = 0;
+    for (size_t i = 0; i < grids.size(); i++) {
+        const GridSize& g = grids[i];
+        if (single || !dev::stepsApply(g.nx, g.ny)) continue;
+        c.stepped[i] = 1;
+        bytes += (int64_t)g.nx * g.ny * size;
+    }
+    if (bytes <= (H == 5 ? kStepBytes5 : kStepBytes3)) {
+        c.stepped.assign(grids.size(), 0);
+        return c;
+    }
+    double least = 0;
+    for (int rows = kStepRows; rows >= 16; rows /= 2) {
+        int64_t waves = 0;
+        for (size_t i = 0; i < grids.size(); i++) {
+            if (!c.stepped[i]) continue;
+            const dev::StepsGrid s = dev::stepsGrid(size, H, grids[i].nx, grids[i].ny, rows);
+            waves += (int64_t)s.strips * s.bands;
+        }
+        const double time = std::max(1.0, (double)waves / kStepSlots + 0.4) *
+                            (rows + dev::kFusedSteps * (H - 1) + 6);
+        if (rows == kStepRows || size == 4 || time < least) {
+            least = time;
+            c.rows = rows;
+        }
+        if (size == 4 && waves >= kStepWaves32) break;
+    }
+    return c;
+}
+
+}  // namespace custen

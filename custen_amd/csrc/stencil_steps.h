@@ -29,6 +29,7 @@
 
 #include <type_traits>
 
+#include "batch_rules.h"
 #include "lds_ring.h"  // row buffers
 #include "stencil_band.h"
 
@@ -37,41 +38,16 @@
 namespace custen {
 namespace dev {
 
-constexpr int kFusedSteps = 3;
-
 template <typename T, int H, int V, int K>
 struct StepsShape {
     static constexpr int D = 8;                          // input rows in flight or in use
-    // columns stored per strip, in whole 64-byte pieces: with 124 and 120 FP32
-    // columns the pass was 10-15 % slower for the lines shared by two strips
-    static constexpr int OW = (kTW - (K - 1) * (H - 1)) / (64 / (int)sizeof(T)) * (64 / (int)sizeof(T));
+    static constexpr int OW = stepsColumns(sizeof(T), H, K);  // columns stored per strip
     static constexpr int HLP = ((H - 1) + 1) & ~1;       // halo columns staged per side
     static constexpr int LD = kTW + 2 * HLP;             // input ring row
     static constexpr int MID = kTW + 2 * HLP;            // row between steps (reads of its unused
                                                          // last columns run on)
     static constexpr int ELEMS = D * LD + (K - 1) * MID;
 };
-
-// Strips and bands of a grid's pass: bands of `rows` rows, at most `most`.
-struct StepsGrid {
-    int strips, bands, rows;
-};
-template <typename T, int H>
-__host__ __device__ inline StepsGrid stepsGrid(int nx, int ny, int most)
-{
-    StepsGrid g;
-    const int ow = StepsShape<T, H, 1, kFusedSteps>::OW;
-    g.strips = (nx + ow - 1) / ow;
-    g.bands = (ny + most - 1) / most;
-    g.rows = (ny + g.bands - 1) / g.bands;
-    return g;
-}
-// One wrap correction must do for every column and row a wave starts at, and a
-// row's bytes for the 31 bits of a buffer's range.
-__host__ __device__ inline bool stepsApply(int nx, int ny)
-{
-    return nx >= kTW && nx < (1 << 28) && ny >= 16;
-}
 
 // Rows that lanes wrote to LDS may be read by other lanes of the wave from here
 // on.  The LDS takes a wave's operations in order, so this costs no
@@ -97,7 +73,7 @@ __device__ __forceinline__ void stepsWalk(const Glob<T>* __restrict__ in, Glob<T
     constexpr int FLAT = sizeof(T) == 8 ? 4 : 2;  // 4-byte loads of a row body
     static_assert((H + 1) % 2 == 0, "pair reads");
     const int lane = threadIdx.x;
-    const StepsGrid sg = stepsGrid<T, H>(nx, ny, most);
+    const StepsGrid sg = stepsGrid(sizeof(T), H, nx, ny, most);
     const int band = __builtin_amdgcn_readfirstlane(g / sg.strips);
     const int strip = g - band * sg.strips;
     const int n = __builtin_amdgcn_readfirstlane(sg.rows);

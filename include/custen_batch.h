@@ -32,12 +32,13 @@ int custenBatchRun(custenBatch* batch, int steps, int mode, hipStream_t stream);
 /* Where the current field of every grid is: 0 = dataInput[g] (before the
  * first step and after an even number of steps), 1 = dataOutput[g]. */
 int custenBatchParity(const custenBatch* batch);
-/* Tile configuration of single fused steps (results do not depend on it):
+/* Tile configuration of the fused steps (results do not depend on it):
  * band = 0: strip kernel, rowsPerWave 4 or 8 and chunks >= 1 row chunks per
  * workgroup; band = 1: band walker (chunks per band) for every grid at least
  * 128 columns wide and a chunk high, strip kernel for the rest.  Replaces the
- * autotuner's choice; graphs captured before are discarded.  Waits for the
- * batch's earlier work on its own stream. */
+ * autotuner's choice, and every step is then a launch of its own, in a batch
+ * that outgrows the L2 caches too; graphs captured before are discarded.  Waits
+ * for the batch's earlier work on its own stream. */
 int custenBatchSetTileConfig(custenBatch* batch, int rowsPerWave, int chunks, int band);
 /* The configuration in use: *band is 1 for the band walker.  All zero before
  * the first fused run when neither the autotuner nor the caller chose one. */

@@ -1,0 +1,42 @@
+"""Which grids of a batch take several steps to a pass over memory (chooseSteps,
+custen_amd/csrc/batch_rules.h), on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = tmp_path_factory.mktemp("rules") / "batch_rules_check"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-I/opt/rocm/include",
+                    os.path.join(HERE, "cpu", "batch_rules_check.cpp"), "-o", str(exe)], check=True)
+
+    def run(*grids, size=8, H=5, single=False):
+        """(rows per band, stepped grids of each group); a group is (count, nx, ny)."""
+        args = ["x".join(map(str, g)) for g in grids]
+        out = subprocess.run([str(exe), str(size), str(H), str(int(single)), *args], check=True,
+                             capture_output=True, text=True).stdout.split()
+        return int(out[0]), [int(v) for v in out[1:]]
+
+    return run
+
+
+@pytest.mark.parametrize("size", [4, 8])
+@pytest.mark.parametrize("H", [3, 5])
+def test_a_batch_that_outgrows_the_caches(choose, size, H):
+    grids = [(8, 2048, 2048), (3, 100, 500), (2, 500, 15)]
+    assert choose(*grids, size=size, H=H)[1] == [8, 0, 0]
+    assert choose((1, 1024, 1024), size=size, H=H)[1] == [0]
+
+
+@pytest.mark.parametrize("size", [4, 8])
+@pytest.mark.parametrize("H", [3, 5])
+def test_a_configured_batch_takes_single_steps(choose, size, H):
+    """The caller's tile configuration says how every step runs."""
+    assert choose((8, 2048, 2048), size=size, H=H, single=True)[1] == [0]
