@@ -35,11 +35,23 @@ __host__ __device__ inline StepsGrid stepsGrid(int size, int H, int nx, int ny, 
     return g;
 }
 
-// One wrap correction must do for every column and row a wave starts at, and a
-// row's bytes for the 31 bits of a buffer's range.
-inline bool stepsApply(int nx, int ny) { return nx >= 128 && nx < (1 << 28) && ny >= 16; }
-
 }  // namespace dev
+
+// The grids that passes are for: one wrap correction must do for every column
+// and row a wave starts at, and a row's bytes for the 31 bits of a buffer's
+// range.  A 5x5 grid of 128 columns takes two strips of a pass for the one of
+// single steps; us per step, passes against single steps, 60 M points:
+//   128 columns, FP64, 16 rows: 215, 164   128: 167, 164   FP32, 16: 124, 88   1000: 101, 85
+//   256 columns, FP64, 16 rows: 167, 169   256: 128, 169   FP32, 16: 93, 92    1000: 92, 92
+//   130 columns, FP64, 64 rows: 169, 269                   FP32, 64: 99, 152
+// and 3x3, which has the FMAs to spare, 128 columns: FP64, 16 rows 118, 160,
+// FP32 82, 84.
+inline bool stepsApply(int size, int H, int nx, int ny)
+{
+    if (nx < 128 || nx >= (1 << 28) || ny < 16) return false;
+    const int single = (nx + 127) / 128;
+    return H == 3 || dev::stepsGrid(size, H, nx, ny, ny).strips < 2 * single;
+}
 
 // Several steps in one pass pay once the two sides no longer stay in the L2s
 // (8 x 4 MiB): single steps then wait for memory, and a pass takes a third of
@@ -81,7 +93,7 @@ inline StepsChoice chooseSteps(const std::vector<GridSize>& grids, int size, int
     int64_t bytes = 0;
     for (size_t i = 0; i < grids.size(); i++) {
         const GridSize& g = grids[i];
-        if (single || !dev::stepsApply(g.nx, g.ny)) continue;
+        if (single || !stepsApply(size, H, g.nx, g.ny)) continue;
         c.stepped[i] = 1;
         bytes += (int64_t)g.nx * g.ny * size;
     }

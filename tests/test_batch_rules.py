@@ -40,3 +40,13 @@ def test_a_batch_that_outgrows_the_caches(choose, size, H):
 def test_a_configured_batch_takes_single_steps(choose, size, H):
     """The caller's tile configuration says how every step runs."""
     assert choose((8, 2048, 2048), size=size, H=H, single=True)[1] == [0]
+
+
+@pytest.mark.parametrize("size", [4, 8])
+def test_grids_whose_strips_double(choose, size):
+    """A 5x5 grid of 128 columns takes two strips of a pass, as many points again
+    as a single step computes."""
+    grids = [(400, 128, 300), (80, 129, 300), (80, 256, 300)]
+    assert choose(*grids, size=size, H=5)[1] == [0, 80, 80]
+    assert choose(*grids, size=size, H=3)[1] == [400, 80, 80]
+    assert choose((1000, 128, 300), size=size, H=5)[1] == [0]
