@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restri
     const int tilesX = (G.nx + kTW - 1) / kTW;
     const int k = item - (rest == 0 ? G.stripBase : rest == 1 ? G.restBase : G.stepsRestBase);
     const int tx = k % tilesX, tyg = k / tilesX;
-    if (stripIsInterior(a, tx)) stencilStripImpl<T, H, V, RPW, Xform::Identity, true>(a, w, tile, tx, tyg);
+    if (stripIsInterior(a, tx, RPW)) stencilStripImpl<T, H, V, RPW, Xform::Identity, true>(a, w, tile, tx, tyg);
     else stencilStripImpl<T, H, V, RPW, Xform::Identity, false>(a, w, tile, tx, tyg);
 }
 

@@ -32,21 +32,23 @@ struct RowMap {
     int rowMax;
 };
 
-// Source row of region row gy for regions at least as tall as the window: one
-// wrap at most for every row that an output of the region needs.  A tile that
-// runs past the region's end holds rows further on, which no stored output
-// needs; the last row stands in for those that one wrap does not bring back
-// (unlimited, a 32-row tile of a grid of 3 rows would be read 26 rows past the
-// array's end).
+// Source row of region row gy where one wrap does.
 __host__ __device__ inline int mapRowNear(const RowMap& m, int gy)
 {
     if (m.wrap) {
-        if (gy < 0) return gy + m.rowWrap;
-        if (gy < m.rowWrap) return gy;
-        gy -= m.rowWrap;
-        return gy < m.rowWrap ? gy : m.rowWrap - 1;
+        if (gy < 0) gy += m.rowWrap;
+        else if (gy >= m.rowWrap) gy -= m.rowWrap;
+        return gy;
     }
     return gy < m.rowMin ? m.rowMin : (gy > m.rowMax ? m.rowMax : gy);
+}
+// Whether one wrap does for every row of the strip kernel's tiles: th rows and a
+// window's T above and B below, the last tile running past the region's ny rows.
+// (Without the second condition a 32-row tile of a periodic grid of 3 rows would
+// be read 26 rows past the array's end.)
+__host__ __device__ inline bool tileRowsNear(const RowMap& m, int ny, int V, int T, int th)
+{
+    return !m.wrap || (m.rowWrap >= V && (ny + th - 1) / th * th + (V - 1 - T) <= 2 * m.rowWrap);
 }
 
 // One stencil apply over a rectangular region of rows [0, ny) of a grid that

@@ -116,14 +116,16 @@ __device__ __forceinline__ void stencilStripImpl(const StencilLaunch& a, const T
 }
 
 // True when column strip tx is a full 128 columns of pair-aligned rows and
-// one wrap suffices for row indices: such strips run the FAST instantiation
-// (only a ragged last strip, or unaligned data, takes the general path).
-__host__ __device__ inline bool stripIsInterior(const StencilLaunch& a, int tx, int cpl = 2)
+// one wrap suffices for row indices (rpw: rows per wave): such strips run the
+// FAST instantiation (only a ragged last strip, unaligned data or a low periodic
+// grid takes the general path).
+__host__ __device__ inline bool stripIsInterior(const StencilLaunch& a, int tx, int rpw,
+                                                int cpl = 2)
 {
     const int tw = kLanes * cpl;
     const int x0 = tx * tw;
     return (cpl == 1 || (a.vecIn && a.vecOut)) && x0 + tw <= a.nx &&
-           (a.rows.wrap ? a.rows.rowWrap >= a.V : true);
+           tileRowsNear(a.rows, a.ny, a.V, a.T, kWaves * rpw);
 }
 
 // Strip g of a single-grid launch -> (tx, tyg): the listed edge strips, or
@@ -143,7 +145,7 @@ __device__ __forceinline__ void stencilStrip(const StencilLaunch& a, const T (&w
 {
     const int tilesX = (a.nx + kTW - 1) / kTW;
     const int tx = g % tilesX, tyg = g / tilesX;
-    if (stripIsInterior(a, tx)) stencilStripImpl<T, H, V, RPW, X, true>(a, w, tile, tx, tyg);
+    if (stripIsInterior(a, tx, RPW)) stencilStripImpl<T, H, V, RPW, X, true>(a, w, tile, tx, tyg);
     else stencilStripImpl<T, H, V, RPW, X, false>(a, w, tile, tx, tyg);
 }
 

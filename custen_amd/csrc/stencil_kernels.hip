@@ -455,10 +455,10 @@ hipError_t runFixed(const StencilLaunch& in, hipStream_t st, KernelUse* use)
     const int rowsPerGroup = dev::kWaves * RPW * s.chunks;
     const int tilesY = (s.ny + rowsPerGroup - 1) / rowsPerGroup;
     int lo = 0, hi = tilesX;  // interior range [lo, hi)
-    while (lo < hi && !dev::stripIsInterior(s, lo, CPL)) lo++;
-    while (hi > lo && !dev::stripIsInterior(s, hi - 1, CPL)) hi--;
+    while (lo < hi && !dev::stripIsInterior(s, lo, RPW, CPL)) lo++;
+    while (hi > lo && !dev::stripIsInterior(s, hi - 1, RPW, CPL)) hi--;
     for (int t = lo; t < hi; t++)
-        if (!dev::stripIsInterior(s, t, CPL)) return hipErrorInvalidValue;  // not contiguous
+        if (!dev::stripIsInterior(s, t, RPW, CPL)) return hipErrorInvalidValue;  // not contiguous
     // edge strips first, one row chunk per workgroup: they are a few percent
     // of the work and must not leave a tail after the interior launch
     const int tilesYe = (s.ny + dev::kWaves * RPW - 1) / (dev::kWaves * RPW);

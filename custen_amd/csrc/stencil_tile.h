@@ -177,10 +177,9 @@ struct StagedRows {
     T halo[2];
 };
 
-// FAST: the strip is a full 128 columns of pair-aligned rows, and the rows that
-// stored outputs need and halo columns take one wrap at most (ny >= window
-// height, nx >= 128 > any extent): no division in the address arithmetic
-// (mapRowNear).
+// FAST: the strip is a full 128 columns of pair-aligned rows, and row and
+// halo-column indices need at most one wrap (tileRowsNear; nx >= 128 > any
+// extent): no division in the address arithmetic.
 template <typename T, int NR, bool FAST, int CPL = 2>
 __device__ __forceinline__ void loadRows(StagedRows<T, NR, CPL>& s, const Glob<T>* __restrict__ in,
                                          int64_t ldIn, const RowMap& rows, int y0, int T_, int x0,
