@@ -31,22 +31,24 @@
 
 namespace custen {
 
+// Items of a batch's launches.  Each kind has a table (owning grid of every item)
+// and each grid its first item of the kind.
+enum ItemKind {
+    kAllStrips = 0,    // every strip
+    kRestStrips = 1,   // with the band walker: strips of the grids it leaves out
+    kBands = 2,        // the band walker's waves
+    kSteps = 3,        // waves of a pass of several steps
+    kStepsRestStrips = 4,  // of the grids such a pass leaves out: strips, or with
+    kStepsRestBands = 5,   // the band walker its waves and the strips of the others
+    kItemKinds = 6
+};
+
 struct BatchDev {
     const void* in;
     void* out;
-    int n;          // nx == ny == n for square grids; nx, ny kept separately below
     int nx, ny;
-    int stripBase;  // first strip id of this grid (strip kernel over all strips)
-    int vec;        // rows pair-aligned
-    // with the band walker: a grid it applies to is walked as a whole, the
-    // others' strips run the strip kernel
-    int walked;
-    int bandBase;   // first band item (wave) of this grid
-    int restBase;   // first strip item of this grid, if it is not walked
-    // passes of several steps: the same for the grids stepsWalk applies to
-    int stepped;
-    int stepsBase;
-    int stepsRestBase;
+    int vec;  // rows pair-aligned
+    int base[kItemKinds];
 };
 
 namespace dev {
@@ -94,16 +96,14 @@ __host__ __device__ __forceinline__ StencilLaunch gridLaunch(const BatchDev& G, 
     return a;
 }
 
-// Strip kernel over every strip of every grid (rest = 0), of the grids that
-// are not walked (1) or of those that passes of several steps leave out (2).
-// itemGrid[item] is the grid that owns the item (built on the host with the
-// item tables, so a workgroup finds its grid with one load).
+// Strip kernel over the strips of a kind.  itemGrid[item] is the grid that owns
+// the item (built on the host, so a workgroup finds its grid with one load).
 template <typename T, int H, int V, int RPW>
 __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restrict__ grids,
                                                         const int* __restrict__ itemGrid,
                                                         int firstItem, int parity,
                                                         const double* __restrict__ weights, int L,
-                                                        int Tt, int chunks, int rest)
+                                                        int Tt, int chunks, ItemKind kind)
 {
     __shared__ __attribute__((aligned(16))) T tile[(kWaves * RPW + V - 1) * ldsRowLength(H)];
     T w[H * V];
@@ -114,19 +114,20 @@ __global__ __launch_bounds__(kThreads) void batchKernel(const BatchDev* __restri
     const StencilLaunch a = gridLaunch(G, parity, sizeof(T) == 8 ? Dtype::F64 : Dtype::F32,
                                        weights, H, L, V, Tt, RPW, chunks);
     const int tilesX = (G.nx + kTW - 1) / kTW;
-    const int k = item - (rest == 0 ? G.stripBase : rest == 1 ? G.restBase : G.stepsRestBase);
+    const int k = item - G.base[kind];
     const int tx = k % tilesX, tyg = k / tilesX;
     if (stripIsInterior(a, tx, RPW)) stencilStripImpl<T, H, V, RPW, Xform::Identity, true>(a, w, tile, tx, tyg);
     else stencilStripImpl<T, H, V, RPW, Xform::Identity, false>(a, w, tile, tx, tyg);
 }
 
-// Band walker over the grids it applies to.
+// Band walker over the items of a kind.
 template <typename T, int H, int V, int RPW>
 __global__ __launch_bounds__(kLanes) void batchBandKernel(const BatchDev* __restrict__ grids,
                                                           const int* __restrict__ itemGrid,
                                                           int parity,
                                                           const double* __restrict__ weights,
-                                                          int L, int Tt, int chunks)
+                                                          int L, int Tt, int chunks,
+                                                          ItemKind kind)
 {
     using BS = BandShape<T, H, V, RPW>;
     __shared__ __attribute__((aligned(16))) T ring[BS::S * BS::LD];
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(kLanes) void batchBandKernel(const BatchDev* __rest
     const BatchDev& G = grids[itemGrid[item]];
     StencilLaunch a = gridLaunch(G, parity, sizeof(T) == 8 ? Dtype::F64 : Dtype::F32, weights, H,
                                  L, V, Tt, RPW, chunks);
-    bandWalk<T, H, V, RPW>(a, w, (Lds<T>*)ring, item - G.bandBase);
+    bandWalk<T, H, V, RPW>(a, w, (Lds<T>*)ring, item - G.base[kind]);
 }
 
 // kFusedSteps steps of the grids stepsWalk applies to.
@@ -157,23 +158,13 @@ __global__ __launch_bounds__(kLanes) void batchStepsKernel(const BatchDev* __res
     const void* in = parity ? G.out : G.in;
     void* out = parity ? const_cast<void*>(G.in) : G.out;
     stepsWalk<T, H, V, kFusedSteps>(globalPtr<T>(in), globalPtr<T>(out), G.nx, G.ny, L, Tt, w,
-                                    (Lds<T>*)lds, most, item - G.stepsBase);
+                                    (Lds<T>*)lds, most, item - G.base[kSteps]);
 }
 
 }  // namespace dev
 }  // namespace custen
 
 using namespace custen;
-
-// Item tables of a batch (owning grid of every item).
-enum ItemKind {
-    kAllStrips = 0,   // every strip
-    kRestStrips = 1,  // strips of the grids the band walker leaves out
-    kBands = 2,       // the band walker's waves
-    kSteps = 3,       // waves of a pass of several steps
-    kStepsRest = 4,   // strips of the grids such a pass leaves out
-    kItemKinds = 5
-};
 
 struct custenBatch {
     int device = 0;
@@ -212,16 +203,17 @@ hipError_t launchOne(const custenBatch* b, int firstItem, int nItems, int parity
                      hipStream_t st)
 {
     const int* owner = b->dItemGrid[kind];
-    if (kind == kBands)
+    if (kind == kBands || kind == kStepsRestBands)
         hipLaunchKernelGGL((dev::batchBandKernel<T, H, V, RPW>), dim3(nItems), dim3(dev::kLanes),
-                           0, st, b->dGrids, owner, parity, b->dWeights, b->L, b->T, b->chunks);
+                           0, st, b->dGrids, owner, parity, b->dWeights, b->L, b->T, b->chunks,
+                           kind);
     else if (kind == kSteps)
         hipLaunchKernelGGL((dev::batchStepsKernel<T, H, V>), dim3(nItems), dim3(dev::kLanes), 0, st,
                            b->dGrids, owner, parity, b->dWeights, b->L, b->T, b->stepRows);
     else
         hipLaunchKernelGGL((dev::batchKernel<T, H, V, RPW>), dim3(nItems), dim3(dev::kThreads), 0,
                            st, b->dGrids, owner, firstItem, parity, b->dWeights, b->L, b->T,
-                           b->chunks, kind == kAllStrips ? 0 : kind == kRestStrips ? 1 : 2);
+                           b->chunks, kind);
     return hipGetLastError();
 }
 
@@ -277,29 +269,27 @@ hipError_t configure(custenBatch* b, int rpw, int chunks, bool band)
         // (what the kernels make of the grid, so that both count the same items)
         const StencilLaunch one = dev::gridLaunch(d, 0, b->dtype, b->dWeights, b->H, b->L, b->V,
                                                   b->T, rpw, chunks);
-        d.walked = band && dev::bandApplies(one, rpw) ? 1 : 0;
-        d.stepped = steps.stepped[i];
-        d.stripBase = (int)n[kAllStrips];
-        d.restBase = (int)n[kRestStrips];
-        d.bandBase = (int)n[kBands];
-        d.stepsBase = (int)n[kSteps];
-        d.stepsRestBase = (int)n[kStepsRest];
+        const bool walked = band && dev::bandApplies(one, rpw);
         const int strips = stripsFor(d.nx, d.ny, rpw, chunks);
         b->strips[i] = strips;
         items[kAllStrips][i] = strips;
-        if (d.walked) {
+        int64_t waves = 0;
+        if (walked) {
             const dev::BandGrid g = dev::bandGrid(one, rpw);
-            items[kBands][i] = (int64_t)g.strips * g.bands;
-        } else if (band) {
-            items[kRestStrips][i] = strips;
+            waves = (int64_t)g.strips * g.bands;
         }
-        if (d.stepped) {
+        if (walked) items[kBands][i] = waves;
+        else if (band) items[kRestStrips][i] = strips;
+        if (steps.stepped[i]) {
             const dev::StepsGrid g = dev::stepsGrid(size, b->H, d.nx, d.ny, steps.rows);
             items[kSteps][i] = (int64_t)g.strips * g.bands;
+        } else if (passes && walked) {
+            items[kStepsRestBands][i] = waves;
         } else if (passes) {
-            items[kStepsRest][i] = strips;
+            items[kStepsRestStrips][i] = strips;
         }
         for (int k = 0; k < kItemKinds; k++) {
+            d.base[k] = (int)n[k];
             n[k] += items[k][i];
             if (n[k] > (int64_t)0x7fffffff) return hipErrorInvalidValue;
         }
@@ -344,8 +334,10 @@ hipError_t enqueueStep(const custenBatch* b, int p, hipStream_t st)
 hipError_t enqueuePass(const custenBatch* b, int p, hipStream_t st)
 {
     hipError_t e = launchAll(b, kSteps, p, st);
-    for (int s = 0; s < dev::kFusedSteps && e == hipSuccess; s++)
-        e = launchAll(b, kStepsRest, (p + s) & 1, st);
+    for (int s = 0; s < dev::kFusedSteps && e == hipSuccess; s++) {
+        e = launchAll(b, kStepsRestBands, (p + s) & 1, st);
+        if (e == hipSuccess) e = launchAll(b, kStepsRestStrips, (p + s) & 1, st);
+    }
     return e;
 }
 
@@ -411,10 +403,8 @@ extern "C" custenBatch* custenBatchCreate(int deviceNum, int numGrids, const int
         BatchDev d{};
         d.in = dataInput[g];
         d.out = dataOutput[g];
-        d.n = nx[g];
         d.nx = nx[g];
         d.ny = ny[g];
-        d.stripBase = (int)strips;
         d.vec = (reinterpret_cast<uintptr_t>(d.in) % (2 * es) == 0 &&
                  reinterpret_cast<uintptr_t>(d.out) % (2 * es) == 0 && nx[g] % 2 == 0)
                     ? 1
@@ -457,7 +447,7 @@ extern "C" int custenBatchRun(custenBatch* b, int steps, int mode, hipStream_t s
         for (int s = 0; s < steps && e == hipSuccess; s++) {
             const int par = (b->parity + s) & 1;
             for (int g = 0; g < b->numGrids && e == hipSuccess; g++)
-                e = launchItems(b, b->host[g].stripBase, b->strips[g], par, st);
+                e = launchItems(b, b->host[g].base[kAllStrips], b->strips[g], par, st);
         }
     } else if (steps > 0) {
         if (!b->tuned && tunerEnabled()) {
