@@ -11,16 +11,19 @@
 // The kernel is bound by its vector instructions, so the flux is written for
 // their number: products by powers of two go into the addition that follows
 // them, and divisions run without the scaling and special cases of IEEE
-// division, which the range of the denominators makes needless; a wave that
-// meets values outside it evaluates that row again operation by operation.
+// division, which the range of the denominators makes needless.  A tile that
+// staged a difference outside that range (kWenoWide) evaluates its points
+// operation by operation instead: 4096 x 4096 with 1 % of the points at 1e9,
+// 185 us, where evaluating a row again after the short forms had left their range
+// took 335 and IEEE divisions throughout 242.
 // Those two forms and the reference's source order with IEEE divisions have the
 // same bits (each shortened step is argued below), so results are bit-identical
 // to the CPU restatement.  Contraction is off; the optional single-precision
 // squares round to float, square in float and widen, as powf does on the
-// reference's double arguments.  4096 x 4096, single-precision squares: 142 us
-// at 91 % of the vector issue rate (240 instructions a point; memory alone would
-// take 100 at the copy rate); with differences and selections per lane and IEEE
-// divisions it took 192.
+// reference's double arguments.  4096 x 4096, single-precision squares: 144 us,
+// the vector unit busy 92 % of the time with 252 instructions a point (memory
+// alone would take 88 at the copy rate); with differences and selections per lane
+// and IEEE divisions it took 192.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -68,7 +71,7 @@ __device__ __forceinline__ double wenoFlux(double v1, double v2, double v3, doub
 }
 
 // n / d with the bits of IEEE division, for a positive normal float d that is
-// 2^120 at most, widened: the reciprocal has 44 good bits after one Newton step
+// 2^125 at most, widened: the reciprocal has 44 good bits after one Newton step
 // from the float estimate, the remainder of the quotient is exact (24 by 53
 // bits), and the quotient's last correction leaves an error of 2^-88, where no
 // quotient by a 24-bit divisor lies within 2^-78 of a rounding boundary.
@@ -96,17 +99,25 @@ __device__ __forceinline__ double quotient(double n, double d)
     return __builtin_fma(__builtin_fma(-d, q, n), y, q);
 }
 
-// wenoFlux with the same bits where `ok` stays true.
-// - x - 2 y and x - 4 y as one fma: the product is exact unless it overflows.
-//   Then either a sum of squares is infinite, which makes the flux NaN here, or
-//   all five differences are that large and nearly equal, and so is the flux.
+// Differences below 2^28 (2^92 where the squares are double) stay in the range of
+// wenoFluxFast: a sum of squares is below 33.4 of their squares, so its own square
+// is below 2^123 (2^380).
+template <bool SS>
+constexpr uint32_t kWenoWide = SS ? 0x41b00000u : 0x45b00000u;  // their high words
+__device__ __forceinline__ uint32_t magnitude(double d)
+{
+    return (uint32_t)(__builtin_bit_cast(uint64_t, d) >> 32) & 0x7fffffffu;
+}
+
+// wenoFlux with the same bits for differences below kWenoWide.
+// - x - 2 y and x - 4 y as one fma: the product is exact.
 // - s + 0.25 b as one fma: the product is exact unless it is subnormal, and 1e-6
 //   is added to the sum.
-// - the squares that divide are 1e-12 at least; the upper end is tested.  The sum
-//   of the quotients is then within the range of the reciprocal's steps.
+// - the squares that divide are 1e-12 at least; the sum of the quotients is then
+//   within the range of the reciprocal's steps.
 template <bool SS>
 __device__ __forceinline__ double wenoFluxFast(double v1, double v2, double v3, double v4,
-                                               double v5, bool& ok)
+                                               double v5)
 {
     const double phi1 = ((1.0 / 3.0) * v1 - (7.0 / 6.0) * v2) + (11.0 / 6.0) * v3;
     const double phi2 = (-(1.0 / 6.0) * v2 + (5.0 / 6.0) * v3) + (1.0 / 3.0) * v4;
@@ -122,13 +133,11 @@ __device__ __forceinline__ double wenoFluxFast(double v1, double v2, double v3, 
     if constexpr (SS) {
         const float f1 = static_cast<float>(s1 + 1e-06), f2 = static_cast<float>(s2 + 1e-06),
                     f3 = static_cast<float>(s3 + 1e-06);
-        ok = ok && __builtin_fmaxf(__builtin_fmaxf(f1, f2), f3) <= 0x1p60f;
         a1 = quotientF(0.1, f1 * f1);
         a2 = quotientF(0.6, f2 * f2);
         a3 = quotientF(0.3, f3 * f3);
     } else {
         const double f1 = s1 + 1e-06, f2 = s2 + 1e-06, f3 = s3 + 1e-06;
-        ok = ok && __builtin_fmax(__builtin_fmax(f1, f2), f3) <= 0x1p190;
         a1 = quotient(0.1, f1 * f1);
         a2 = quotient(0.6, f2 * f2);
         a3 = quotient(0.3, f3 * f3);
@@ -137,9 +146,7 @@ __device__ __forceinline__ double wenoFluxFast(double v1, double v2, double v3, 
     const double y = recipOf(sum);
     const double denom = __builtin_fma(__builtin_fma(-sum, y, 1.0), y, y);
     const double w1 = a1 * denom, w2 = a2 * denom, w3 = a3 * denom;
-    const double flux = (phi1 * w1 + phi2 * w2) + phi3 * w3;
-    ok = ok && __builtin_fabs(flux) <= 0x1p1000;
-    return flux;
+    return (phi1 * w1 + phi2 * w2) + phi3 * w3;
 }
 
 template <int RPW, bool SS>
@@ -151,6 +158,7 @@ __global__ __launch_bounds__(kThreads) void wenoKernel(WenoLaunch a, int tilesX,
     // y differences: row r is (q(y0 - 2 + r) - q(y0 - 3 + r)) / dy
     __shared__ double diffX[TH * kWenoLX];
     __shared__ double diffY[(TH + 5) * kWenoTW];
+    __shared__ int wideWave[kWaves];  // the wave staged a difference that is kWenoWide or more
 
     const int g = xcdRemap(blockIdx.x, gridDim.x);
     // g / tilesX from the rounded-down reciprocal, at most one too small
@@ -204,40 +212,54 @@ __global__ __launch_bounds__(kThreads) void wenoKernel(WenoLaunch a, int tilesX,
         uv[k] = rowLoad(rowBuffer(a.u + at), here);
         vv[k] = rowLoad(rowBuffer(a.v + at), here);
     }
+    uint32_t most = 0;
+    auto stage = [&](double* at, double d) {
+        *at = d;
+        most = max(most, magnitude(d));
+    };
 #pragma unroll
     for (int k = 0; k < PER; k++)
-        if (rBegin + k < TH + 5) diffY[(rBegin + k) * kWenoTW + lane] = (q[k + 1] - q[k]) * a.coeDy;
+        if (rBegin + k < TH + 5)
+            stage(diffY + (rBegin + k) * kWenoTW + lane, (q[k + 1] - q[k]) * a.coeDy);
 #pragma unroll
     for (int k = 0; k < RPW; k++)
-        diffX[(wave * RPW + k) * kWenoLX + lane] = (qa[k] - qb[k]) * a.coeDx;
-    if (lane < 5 * RPW) diffX[(wave * RPW + tr) * kWenoLX + kWenoTW + tc] = (ta - tb) * a.coeDx;
+        stage(diffX + (wave * RPW + k) * kWenoLX + lane, (qa[k] - qb[k]) * a.coeDx);
+    if (lane < 5 * RPW)
+        stage(diffX + (wave * RPW + tr) * kWenoLX + kWenoTW + tc, (ta - tb) * a.coeDx);
+    wideWave[wave] = __ballot(most >= kWenoWide<SS>) != 0;
     __syncthreads();
+    int wide = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; k++) wide |= wideWave[k];
+    wide = __builtin_amdgcn_readfirstlane(wide);
 
     const int x = x0 + lane;
     if (x >= a.nx) return;
+    auto rows = [&](auto flux) {
 #pragma unroll
-    for (int r = 0; r < RPW; r++) {
-        const int ly = wave * RPW + r;
-        const int y = y0 + ly;
-        if (y >= a.ny) break;
-        // the middle one of the five differences, and the way to the others
-        const bool px = uv[r] > 0.0, py = vv[r] > 0.0;
-        const double* mx = diffX + ly * kWenoLX + lane + (px ? 2 : 3);
-        const double* my = diffY + (ly + (py ? 2 : 3)) * kWenoTW + lane;
-        const int sx = px ? 1 : -1, sy = py ? kWenoTW : -kWenoTW;
-        double dx[5] = {mx[-2 * sx], mx[-sx], mx[0], mx[sx], mx[2 * sx]};
-        double dy[5] = {my[-2 * sy], my[-sy], my[0], my[sy], my[2 * sy]};
-        bool ok = true;
-        double fx = wenoFluxFast<SS>(dx[0], dx[1], dx[2], dx[3], dx[4], ok);
-        double fy = wenoFluxFast<SS>(dy[0], dy[1], dy[2], dy[3], dy[4], ok);
-        if (__builtin_expect(__ballot(!ok) != 0, 0)) {
-            // (taken from here on, so that it is not computed beside the other)
-            __asm__ __volatile__("" : "+v"(dx[0]), "+v"(dx[1]), "+v"(dx[2]), "+v"(dx[3]), "+v"(dx[4]));
-            __asm__ __volatile__("" : "+v"(dy[0]), "+v"(dy[1]), "+v"(dy[2]), "+v"(dy[3]), "+v"(dy[4]));
-            fx = wenoFlux<SS>(dx[0], dx[1], dx[2], dx[3], dx[4]);
-            fy = wenoFlux<SS>(dy[0], dy[1], dy[2], dy[3], dy[4]);
+        for (int r = 0; r < RPW; r++) {
+            const int ly = wave * RPW + r;
+            const int y = y0 + ly;
+            if (y >= a.ny) break;
+            // the middle one of the five differences, and the way to the others
+            const bool px = uv[r] > 0.0, py = vv[r] > 0.0;
+            const double* mx = diffX + ly * kWenoLX + lane + (px ? 2 : 3);
+            const double* my = diffY + (ly + (py ? 2 : 3)) * kWenoTW + lane;
+            const int sx = px ? 1 : -1, sy = py ? kWenoTW : -kWenoTW;
+            const double fx = flux(mx[-2 * sx], mx[-sx], mx[0], mx[sx], mx[2 * sx]);
+            const double fy = flux(my[-2 * sy], my[-sy], my[0], my[sy], my[2 * sy]);
+            __builtin_nontemporal_store(uv[r] * fx + vv[r] * fy,
+                                        a.out + (int64_t)y * a.ldOut + x);
         }
-        __builtin_nontemporal_store(uv[r] * fx + vv[r] * fy, a.out + (int64_t)y * a.ldOut + x);
+    };
+    if (__builtin_expect(wide, 0)) {
+        rows([](double v1, double v2, double v3, double v4, double v5) {
+            return wenoFlux<SS>(v1, v2, v3, v4, v5);
+        });
+    } else {
+        rows([](double v1, double v2, double v3, double v4, double v5) {
+            return wenoFluxFast<SS>(v1, v2, v3, v4, v5);
+        });
     }
 }
 
@@ -263,7 +285,8 @@ int wenoLdsBytes(int rowsPerWave)
 {
     const int rpw = rowsPerWave == 8 ? 8 : 4;
     const int rows = dev::kWaves * rpw;
-    return (rows * dev::kWenoLX + (rows + 5) * dev::kWenoTW) * (int)sizeof(double);
+    return (rows * dev::kWenoLX + (rows + 5) * dev::kWenoTW) * (int)sizeof(double) +
+           dev::kWaves * (int)sizeof(int);
 }
 
 hipError_t launchWeno(const WenoLaunch& w, hipStream_t st)
