@@ -250,6 +250,7 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
         const __amdgpu_buffer_rsrc_t rl = dev::rowBuffer(dl + at), rd = dev::rowBuffer(d + at),
                                      ru = dev::rowBuffer(du + at), rw = dev::rowBuffer(dw + at);
         const double duPPs = duPP, dwPPs = dwPP, duPs = duP, dwPs = dwP;
+        double vl[CR], vd[CR], vu[CR], vw[CR];
         double qmin = 0x1p900, dmin = 0x1p900, dmax = 0.0;
 #pragma unroll
         for (int j = 0; j < CR; j++) {
@@ -261,11 +262,10 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
             qmin = __builtin_fmin(qmin, __builtin_fmin(__builtin_fabs(uv), __builtin_fabs(wv)));
             dmin = __builtin_fmin(dmin, __builtin_fabs(dv));
             dmax = __builtin_fmax(dmax, __builtin_fabs(dv));
-            const uint32_t o = (uint32_t)j * stride;
-            dev::rowStore(rl, lv, col8, o);
-            dev::rowStore(rd, dv, col8, o);
-            dev::rowStore(ru, uv, col8, o);
-            dev::rowStore(rw, wv, col8, o);
+            vl[j] = lv;
+            vd[j] = dv;
+            vu[j] = uv;
+            vw[j] = wv;
             duPP = duP;
             dwPP = dwP;
             duP = uv;
@@ -281,20 +281,27 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
             dwP = dwPs;
 #pragma unroll
             for (int j = 0; j < CR; j++) {
-                const double lv = x[1][j] - x[0][j] * duPP;
-                const double dv = (x[2][j] - x[0][j] * dwPP) - lv * duP;
-                const double uv = (x[3][j] - lv * dwP) / dv;
-                const double wv = x[4][j] / dv;
-                const uint32_t o = (uint32_t)j * stride;
-                dev::rowStore(rl, lv, col8, o);
-                dev::rowStore(rd, dv, col8, o);
-                dev::rowStore(ru, uv, col8, o);
-                dev::rowStore(rw, wv, col8, o);
+                vl[j] = x[1][j] - x[0][j] * duPP;
+                vd[j] = (x[2][j] - x[0][j] * dwPP) - vl[j] * duP;
+                vu[j] = (x[3][j] - vl[j] * dwP) / vd[j];
+                vw[j] = x[4][j] / vd[j];
                 duPP = duP;
                 dwPP = dwP;
-                duP = uv;
-                dwP = wv;
+                duP = vu[j];
+                dwP = vw[j];
             }
+        }
+        // A chunk's rows are stored once, when they are right: stored again after
+        // such a chunk they cost as much as the divisions (a zero above the
+        // diagonal in every third row, us: 24576 systems 416, and 538 so; the
+        // one-wave kernel 501).
+#pragma unroll
+        for (int j = 0; j < CR; j++) {
+            const uint32_t o = (uint32_t)j * stride;
+            dev::rowStore(rl, vl[j], col8, o);
+            dev::rowStore(rd, vd[j], col8, o);
+            dev::rowStore(ru, vu[j], col8, o);
+            dev::rowStore(rw, vw[j], col8, o);
         }
     };
     Rows<5> A, B;
@@ -780,8 +787,8 @@ int check(const char* fn, const void* const* ptrs, int nptr, int m, int batchCou
 }
 
 // Where the ring kernels are the faster ones (us at 1022 rows, one-wave kernel
-// -> ring kernel): a factorisation of 4096 systems 344 -> 125, 16384 404 ->
-// 205, 32768 523 -> 443, 40960 645 -> 613, 49152 667 -> 709; a solve of 4096
+// -> ring kernel): a factorisation of 4096 systems 342 -> 120, 16384 398 ->
+// 213, 32768 520 -> 443, 40960 638 -> 618, 49152 667 -> 709; a solve of 4096
 // 262 -> 131, 16384 358 -> 244, 20480 431 -> 432, 32768 476 -> 504.  Above
 // the limits the one-wave kernel has several waves on every SIMD and runs at
 // the memory's rate, while the ring kernel has one workgroup on a CU.
