@@ -788,11 +788,12 @@ int check(const char* fn, const void* const* ptrs, int nptr, int m, int batchCou
 
 // Where the ring kernels are the faster ones (us at 1022 rows, one-wave kernel
 // -> ring kernel): a factorisation of 4096 systems 342 -> 120, 16384 398 ->
-// 213, 32768 520 -> 443, 40960 638 -> 618, 49152 667 -> 709; a solve of 4096
-// 262 -> 131, 16384 358 -> 244, 20480 431 -> 432, 32768 476 -> 504.  Above
-// the limits the one-wave kernel has several waves on every SIMD and runs at
-// the memory's rate, while the ring kernel has one workgroup on a CU.
-constexpr int kFactorRingMax = 40960;
+// 213, 32768 520 -> 443, 40960 638 -> 618; a solve of 4096 262 -> 131, 16384 358
+// -> 244, 20480 431 -> 432, 32768 476 -> 504.  Above the limits the one-wave
+// kernel has several waves on every SIMD and runs at the memory's rate, while the
+// ring kernel has one workgroup on a CU, and short systems lose in its third
+// round (factorisation of 40960: 32 rows 22.3 -> 27.9, 64 rows 39.5 -> 44.7).
+constexpr int kFactorRingMax = 32768;
 constexpr int kSolveRingMax = 16384;
 // A solve of few systems takes 16 per workgroup, so that four times as many CUs
 // fetch (their outstanding loads are what a CU's share of a sweep waits for):
