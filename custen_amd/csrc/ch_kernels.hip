@@ -308,7 +308,8 @@ __device__ __forceinline__ double divByRecip(double n, double d, double y)
     return __builtin_fma(__builtin_fma(-d, q, n), y, q);
 }
 // An infinity or NaN stays in the recurrence to the end of a step, where its
-// last value shows it (the factors of the value before are not 0).
+// last value shows it: a factor of the value before makes it an infinity or NaN
+// again, or NaN where the factor is 0, and nothing finite comes of that.
 __device__ __forceinline__ bool isFinite(double v) { return __builtin_fabs(v) < __builtin_inf(); }
 
 // v of lane i (the same for all lanes).
@@ -428,8 +429,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
 #pragma unroll
             for (int k = 0; k < SR; k++) buf[k] = load(p, k);
         };
-        // every row of the staged step has a reciprocal, and a factor of the
-        // row before (uniform)
+        // every row of the staged step has a reciprocal (uniform)
         bool recips = true;
         auto stageDiag = [&](int slot, double p0, double p1, double p2) {
             const double y = divRecip(p2);
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             sd[slot][1][lane] = p1;
             sd[slot][2][lane] = p2;
             sd[slot][3][lane] = y;
-            recips = __all(y != 0.0 && p1 != 0.0);
+            recips = __all(y != 0.0);
         };
         auto diagRow = [&](int j) { return min(2 + j * SR + min(lane, SR - 1), m - 1); };
         // step j: diagonals of step j+1 and the column rows of step j+2 are
@@ -487,10 +487,9 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             stageDiag(slot ^ 1, p0, p1, p2);
         };
         // a step inside the constant run; `fast`: the pivot is certified for
-        // the two-operation division q = fma(x, ky, RN(x kz)) = RN(x / k2)
-        // (2^-900 <= |x| <= 2^900), kz the low part of 1/k2
+        // the two-operation division q = fma(x, ky, RN(x kz)) = RN(x / k2) (|x| >=
+        // 2^-900; where x / k2 overflows so does q), kz the low part of 1/k2
         double kz = 0.0;
-        const bool short2 = ky != 0.0 && k1 != 0.0;
         auto stepK = [&](auto fast, int j, const double (&cur)[SR], double (&ahead)[SR],
                         const __amdgpu_buffer_rsrc_t& out, __amdgpu_buffer_rsrc_t& outAhead) {
             loadStep(ahead, outAhead, j + 2);
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 b2 = b1;
                 b1 = v;
             }
-            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && short2), 0)) {
+            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && ky != 0.0), 0)) {
                 b2 = b2s;
                 b1 = b1s;
                 for (int k = 0; k < SR; k++) {

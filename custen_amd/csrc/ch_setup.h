@@ -112,10 +112,12 @@ CUSTEN_CH_HD inline void chConstantRuns(const double* fac, int m, int& fwd, int&
 // M = -(e / 2^s) Do^-1 modulo 2^(P-s): a handful of (M, X) per e.
 //
 // Scaling x and d by powers of two changes nothing while no operation
-// underflows or overflows; the kernels use the result only for
-// 2^-900 <= |x| <= 2^900 and 2^-60 <= |d| <= 2^60, where that holds (an
-// RN(x zl) in the subnormal range adds at most 2^-1075, far inside the margin
-// of the wider e range).  Signs are symmetric.
+// underflows or overflows.  The kernels use the result for |x| >= 2^-900 and
+// 2^-60 <= |d| <= 2^60, where none underflows (an RN(x zl) in the subnormal range
+// adds at most 2^-1075, far inside the margin of the wider e range), and for x up
+// to the largest: x zl and the sum overflow only where x / d does, which leaves
+// an infinity or NaN; the kernels divide again by IEEE division where a step ends
+// with one (tests/cpu/division_top_check.cpp).  Signs are symmetric.
 // ---------------------------------------------------------------------------
 namespace chdiv {
 
@@ -194,7 +196,7 @@ CUSTEN_CH_HD inline bool certified(T d)
 
 // The divisor d of the column solve's constant run may use the two-operation
 // division (q = fma(x, zh, x zl) with zh = RN(1/d), zl = RN(fma(-d, zh, 1) / d))
-// for 2^-900 <= |x| <= 2^900.
+// for |x| >= 2^-900, as far as x / d is finite.
 CUSTEN_CH_HD inline bool chDivCertified(double d)
 {
     const double ad = d < 0 ? -d : d;
