@@ -472,8 +472,10 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
             }
             // a numerator outside divByRecip's range (zero, whose sign the
             // corrections would lose, subnormal, Inf) or a row without a
-            // reciprocal: this lane repeats the step with IEEE division
-            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && recips), 0)) {
+            // reciprocal: this lane repeats the step with IEEE division (after a
+            // NaN all is NaN either way)
+            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && recips), 0) &&
+                b1s == b1s) {
                 b2 = b2s;
                 b1 = b1s;
                 for (int k = 0; k < SR; k++) {
@@ -508,7 +510,8 @@ __global__ __launch_bounds__(64, 2) void colSolveKernel(const CHDesc* __restrict
                 b2 = b1;
                 b1 = v;
             }
-            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && ky != 0.0), 0)) {
+            if (__builtin_expect(!(nmin >= 0x1p-900 && isFinite(b1) && ky != 0.0), 0) &&
+                b1s == b1s) {
                 b2 = b2s;
                 b1 = b1s;
                 for (int k = 0; k < SR; k++) {
