@@ -20,6 +20,7 @@
 #include "../../include/custen_pent.h"
 #include "lds_ring.h"
 #include "plan_internal.h"
+#include "short_division.h"
 
 #pragma clang fp contract(off)
 
@@ -45,7 +46,12 @@ constexpr int kBlock = 64;
 // ---------------------------------------------------------------------------
 constexpr int CR = 8;  // rows per chunk
 
+using dev::kMaxDivisor;
+using dev::kMinDivisor;
+using dev::kMinQuotient;
 using dev::Lds;
+using dev::quotient;
+using dev::recipOf;
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 struct __attribute__((aligned(16))) Progress {
@@ -175,25 +181,6 @@ __device__ __forceinline__ void readChunk(double (&r)[N][CR], const Lds<char>* r
 #pragma unroll
         for (int k = 0; k < CR; k++) r[a][k] = p[a * (RG::ARRAY / 8) + k * (RG::ROW / 8)];
 }
-
-// Division by a value whose reciprocal is at hand: the steps of the GPU's IEEE
-// division (reciprocal estimate, two Newton steps, quotient, remainder, one
-// correction) without its operand scaling and special-case fixup, which leave
-// operands alone while |d| lies in [2^-500, 2^500] and the quotient in
-// [2^-400, finite]; within that range the bits are those of n / d.
-__device__ __forceinline__ double recipOf(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-    return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-}
-__device__ __forceinline__ double quotient(double n, double d, double y)
-{
-    const double q = n * y;
-    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
-}
-constexpr double kMinQuotient = 0x1p-400;
-constexpr double kMinDivisor = 0x1p-500, kMaxDivisor = 0x1p500;
 
 // pentFactorBatch (cuPentBatch.cu:35-113)
 template <int SYS, int BYTES>

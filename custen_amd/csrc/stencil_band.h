@@ -18,12 +18,12 @@
 // Every point of a walked strip is written, so there are no store masks: the
 // walked strips tile the written columns of the launch, the last one ending
 // at the last written column (it overlaps its neighbour, and so may the first,
-// when the window is not made of whole strips), and the chunks tile the written rows, the last band
-// ending at the last of them.  Points in an overlap are computed by both
+// when the window is not made of whole strips), and the chunks tile the written
+// rows, the last band ending at the last of them.  Points in an overlap are computed by both
 // waves from the same values in the same order.  A strip may start at any
 // column and rows at any alignment of an element: the loads and stores need
 // element alignment only.  At 4099 x 3001 (5x5, FP64, written window inside a
-// one-cell border on odd rows) the apply takes 32.0 us (197 MB, 6.1
+// two-cell border, odd rows) the apply takes 32.0 us (197 MB, 6.1
 // TB/s), against 49.4 when such rows took the strip kernel's per-element path.
 //
 // Arithmetic is the fma chain of the other stencil kernels (row j outer,
@@ -91,6 +91,12 @@ __device__ __forceinline__ void ldsDma4(const Glob<unsigned>* g, Lds<T>* l)
     __builtin_amdgcn_global_load_lds((const Glob<void>*)g, (LdsVoid*)l, 4, 0, POLICY);
 }
 
+// A pair of elements at element alignment.
+template <typename T> struct ElemPair;
+template <> struct ElemPair<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct ElemPair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <typename T> using ElemVec2 = typename ElemPair<T>::type;
+
 // FP64 stencils of more than 36 points have more weights than the scalar
 // registers hold next to the walker's own state; held for the whole walk they
 // are spilled and read back lane by lane.  The walk of those stencils instead
@@ -103,12 +109,6 @@ constexpr bool kStreamWeights = sizeof(T) == 8 && H * V > 36;
 // FP32 stencils of more than 36 points: the weights (converted from the
 // FP64 array on the vector unit) stay in vector registers, 49 or 81 of them,
 // instead of being moved to scalar registers that then spill.
-// A pair of elements at element alignment.
-template <typename T> struct ElemPair;
-template <> struct ElemPair<double> { typedef double type __attribute__((ext_vector_type(2), aligned(8))); };
-template <> struct ElemPair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
-template <typename T> using ElemVec2 = typename ElemPair<T>::type;
-
 template <typename T, int H, int V>
 constexpr bool kWeightsInVgprs = sizeof(T) == 4 && H * V > 36;
 

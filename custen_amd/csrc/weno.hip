@@ -28,6 +28,7 @@
 
 #include "kernels.h"
 #include "lds_ring.h"  // row buffers
+#include "short_division.h"
 #include "stencil_tile.h"
 
 #pragma clang fp contract(off)
@@ -83,22 +84,6 @@ __device__ __forceinline__ double quotientF(double n, float d)
     const double q = n * y;
     return __builtin_fma(__builtin_fma(-w, q, n), y, q);
 }
-// The steps of the GPU's IEEE division without operand scaling and fixup, which
-// leave operands alone for divisors in [2^-500, 2^500] and quotients of at least
-// 2^-400.
-__device__ __forceinline__ double recipOf(double d)
-{
-    double y = __builtin_amdgcn_rcp(d);
-    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-    return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-}
-__device__ __forceinline__ double quotient(double n, double d)
-{
-    const double y = recipOf(d);
-    const double q = n * y;
-    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
-}
-
 // Differences below 2^28 (2^92 where the squares are double) stay in the range of
 // wenoFluxFast: a sum of squares is below 33.4 of their squares, so its own square
 // is below 2^123 (2^380).
@@ -138,9 +123,10 @@ __device__ __forceinline__ double wenoFluxFast(double v1, double v2, double v3, 
         a3 = quotientF(0.3, f3 * f3);
     } else {
         const double f1 = s1 + 1e-06, f2 = s2 + 1e-06, f3 = s3 + 1e-06;
-        a1 = quotient(0.1, f1 * f1);
-        a2 = quotient(0.6, f2 * f2);
-        a3 = quotient(0.3, f3 * f3);
+        const double g1 = f1 * f1, g2 = f2 * f2, g3 = f3 * f3;
+        a1 = quotient(0.1, g1, recipOf(g1));
+        a2 = quotient(0.6, g2, recipOf(g2));
+        a3 = quotient(0.3, g3, recipOf(g3));
     }
     const double sum = (a1 + a2) + a3;
     const double y = recipOf(sum);
