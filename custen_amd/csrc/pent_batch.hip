@@ -182,8 +182,10 @@ __device__ __forceinline__ void readChunk(double (&r)[N][CR], const Lds<char>* r
         for (int k = 0; k < CR; k++) r[a][k] = p[a * (RG::ARRAY / 8) + k * (RG::ROW / 8)];
 }
 
-// pentFactorBatch (cuPentBatch.cu:35-113)
-template <int SYS, int BYTES>
+// pentFactorBatch (cuPentBatch.cu:35-113).  LATE: a chunk's rows are stored when
+// its quotients are known to be in the short division's range, and then once;
+// otherwise as they are computed, and again after a chunk that left it.
+template <int SYS, int BYTES, bool LATE>
 __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
                                                         double* __restrict__ dl,
                                                         double* __restrict__ d,
@@ -238,6 +240,13 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
                                      ru = dev::rowBuffer(du + at), rw = dev::rowBuffer(dw + at);
         const double duPPs = duPP, dwPPs = dwPP, duPs = duP, dwPs = dwP;
         double vl[CR], vd[CR], vu[CR], vw[CR];
+        auto storeRow = [&](int j) {
+            const uint32_t o = (uint32_t)j * stride;
+            dev::rowStore(rl, vl[j], col8, o);
+            dev::rowStore(rd, vd[j], col8, o);
+            dev::rowStore(ru, vu[j], col8, o);
+            dev::rowStore(rw, vw[j], col8, o);
+        };
         double qmin = 0x1p900, dmin = 0x1p900, dmax = 0.0;
 #pragma unroll
         for (int j = 0; j < CR; j++) {
@@ -253,6 +262,7 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
             vd[j] = dv;
             vu[j] = uv;
             vw[j] = wv;
+            if constexpr (!LATE) storeRow(j);
             duPP = duP;
             dwPP = dwP;
             duP = uv;
@@ -272,23 +282,16 @@ __global__ __launch_bounds__(192) void factorRingKernel(double* __restrict__ ds,
                 vd[j] = (x[2][j] - x[0][j] * dwPP) - vl[j] * duP;
                 vu[j] = (x[3][j] - vl[j] * dwP) / vd[j];
                 vw[j] = x[4][j] / vd[j];
+                if constexpr (!LATE) storeRow(j);
                 duPP = duP;
                 dwPP = dwP;
                 duP = vu[j];
                 dwP = vw[j];
             }
         }
-        // A chunk's rows are stored once, when they are right: stored again after
-        // such a chunk they cost as much as the divisions (a zero above the
-        // diagonal in every third row, us: 24576 systems 416, and 538 so; the
-        // one-wave kernel 501).
+        if constexpr (LATE) {
 #pragma unroll
-        for (int j = 0; j < CR; j++) {
-            const uint32_t o = (uint32_t)j * stride;
-            dev::rowStore(rl, vl[j], col8, o);
-            dev::rowStore(rd, vd[j], col8, o);
-            dev::rowStore(ru, vu[j], col8, o);
-            dev::rowStore(rw, vw[j], col8, o);
+            for (int j = 0; j < CR; j++) storeRow(j);
         }
     };
     Rows<5> A, B;
@@ -781,6 +784,13 @@ int check(const char* fn, const void* const* ptrs, int nptr, int m, int batchCou
 // ring kernel has one workgroup on a CU, and short systems lose in its third
 // round (factorisation of 40960: 32 rows 22.3 -> 27.9, 64 rows 39.5 -> 44.7).
 constexpr int kFactorRingMax = 32768;
+// Rows stored late cost nothing (4096 systems 122 -> 120 us, 24576 389 -> 388) and
+// spare a chunk with a zero quotient its second stores (a zero above the diagonal
+// in every third row, us: 24576 systems 538 -> 412, where the one-wave kernel
+// takes 501), but where rows are not 16-byte aligned and workgroups few, the
+// burst of stores is waited for (898 rows, 245 systems 102.8 -> 108.0, 4095
+// 107.3 -> 109.5, 8191 164.9 -> 162.7).
+constexpr int kFactorEarlyMax = 4096;
 constexpr int kSolveRingMax = 16384;
 // A solve of few systems takes 16 per workgroup, so that four times as many CUs
 // fetch (their outstanding loads are what a CU's share of a sweep waits for):
@@ -814,11 +824,14 @@ extern "C" int custenPentFactorBatch(double* ds, double* dl, double* d, double* 
         hipLaunchKernelGGL(pentdev::factorKernel, dim3(blocksOf(n, pentdev::kBlock)),
                            dim3(pentdev::kBlock), 0, stream, ds, dl, d, du, dw, m, n);
     else if (wideRows(ptrs, 5, batchCount))
-        hipLaunchKernelGGL((pentdev::factorRingKernel<64, 16>), dim3(blocksOf(n, 64)), dim3(192), 0,
-                           stream, ds, dl, d, du, dw, m, n);
+        hipLaunchKernelGGL((pentdev::factorRingKernel<64, 16, true>), dim3(blocksOf(n, 64)),
+                           dim3(192), 0, stream, ds, dl, d, du, dw, m, n);
+    else if (batchCount > kFactorEarlyMax)
+        hipLaunchKernelGGL((pentdev::factorRingKernel<64, 4, true>), dim3(blocksOf(n, 64)),
+                           dim3(192), 0, stream, ds, dl, d, du, dw, m, n);
     else
-        hipLaunchKernelGGL((pentdev::factorRingKernel<64, 4>), dim3(blocksOf(n, 64)), dim3(192), 0,
-                           stream, ds, dl, d, du, dw, m, n);
+        hipLaunchKernelGGL((pentdev::factorRingKernel<64, 4, false>), dim3(blocksOf(n, 64)),
+                           dim3(192), 0, stream, ds, dl, d, du, dw, m, n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         setHipError(e, "custenPentFactorBatch");

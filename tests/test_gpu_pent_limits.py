@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m", [4, 13, 35])
-@pytest.mark.parametrize("batch", [8192, 8193, 16384, 16385, 16386, 32767, 32768, 32769, 32770])
+@pytest.mark.parametrize("batch", [4095, 4097, 8192, 8193, 16384, 16385, 16386, 32767, 32768, 32769, 32770])
 def test_around_the_limits(gpu, m, batch):
     print(f"pent limits m={m} batch={batch}", flush=True)
     host = _pent_systems(m, batch, m + batch)

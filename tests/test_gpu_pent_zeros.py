@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("zero", [0.0, -0.0])
 @pytest.mark.parametrize("sign", [1.0, -1.0])
 @pytest.mark.parametrize("which", ["dw", "du", "du dw", "ds dw", "ds dl du dw", "some rows"])
-@pytest.mark.parametrize("m,batch", [(45, 96), (67, 65)])
+@pytest.mark.parametrize("m,batch", [(45, 96), (67, 65), (30, 4099)])
 def test_zero_quotients(gpu, which, sign, zero, m, batch):
     print(f"pent zeros {which} {sign} {zero} m={m} batch={batch}", flush=True)
     host = [a * sign for a in _pent_systems(m, batch, 3 * m)]
