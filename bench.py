@@ -783,8 +783,8 @@ def bench_stream(args, extra=None):
                                      ref[1:4, 1:-1].view(np.uint64)))
     res["mismatching_points_sampled_rows"] = mism
     # host link ceilings: 1 GiB each way alone, and both ways at once on two
-    # streams (the aggregate bounds a streamed apply, which moves the field in
-    # and the result out)
+    # streams (copies of this size take turns on the link; the aggregate bounds a
+    # streamed apply whose tiles are as large)
     n1 = (1 << 30) // 8
     dev_a = torch.empty(n1, dtype=torch.float64, device="cuda")
     dev_b = torch.zeros(n1, dtype=torch.float64, device="cuda")
