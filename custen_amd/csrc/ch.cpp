@@ -22,7 +22,6 @@
 #include <map>
 #include <memory>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -31,6 +30,7 @@
 #include "ch_kernels.h"
 #include "ch_plain.h"
 #include "ch_setup.h"
+#include "host_copy.h"
 #include "plan_internal.h"
 
 #pragma STDC FP_CONTRACT OFF
@@ -1310,41 +1310,6 @@ extern "C" int custenCHServerQuery(custenCHServer* s, int id, int* state, double
     }
     return CUSTEN_SUCCESS;
 }
-
-namespace {
-
-// Host copy of a result into the caller's array.  A copy into memory the caller
-// has not touched yet is bound by page faults (2 MB take 0.9 ms), which the
-// kernel serves in parallel: it is split over up to 8 threads, with 512 KB each
-// at least.
-void copyOut(double* dst, const double* src, size_t count)
-{
-    constexpr size_t kSplitBytes = size_t(512) << 10;
-    const unsigned hw = std::thread::hardware_concurrency();
-    const size_t parts = std::min({count * sizeof(double) / kSplitBytes, (size_t)hw, (size_t)8});
-    if (parts <= 1) {
-        std::memcpy(dst, src, count * sizeof(double));
-        return;
-    }
-    const size_t chunk = (count + parts - 1) / parts;
-    std::thread workers[8];
-    size_t rest = count;  // where the workers' parts begin
-    try {
-        for (size_t t = parts - 1; t > 0; t--) {
-            const size_t b = t * chunk, e = rest;
-            if (b >= e) continue;
-            workers[t] = std::thread([=]() { std::memcpy(dst + b, src + b, (e - b) * sizeof(double)); });
-            rest = b;
-        }
-    } catch (const std::system_error&) {
-        // no more threads: the rest is copied here
-    }
-    std::memcpy(dst, src, rest * sizeof(double));
-    for (std::thread& w : workers)
-        if (w.joinable()) w.join();
-}
-
-}  // namespace
 
 extern "C" int custenCHServerResult(custenCHServer* s, int id, double* c)
 {
