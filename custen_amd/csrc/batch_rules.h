@@ -39,18 +39,22 @@ __host__ __device__ inline StepsGrid stepsGrid(int size, int H, int nx, int ny, 
 
 // The grids that passes are for: one wrap correction must do for every column
 // and row a wave starts at, and a row's bytes for the 31 bits of a buffer's
-// range.  A 5x5 grid of 128 columns takes two strips of a pass for the one of
-// single steps; us per step, passes against single steps, 60 M points:
+// range.
+inline bool stepsApply(int nx, int ny) { return nx >= 128 && nx < (1 << 28) && ny >= 16; }
+
+// A 5x5 grid of 128 columns takes two strips of a pass for the one of single
+// steps; us per step, passes against single steps, 60 M points:
 //   128 columns, FP64, 16 rows: 215, 164   128: 167, 164   FP32, 16: 124, 88   1000: 101, 85
 //   256 columns, FP64, 16 rows: 167, 169   256: 128, 169   FP32, 16: 93, 92    1000: 92, 92
 //   130 columns, FP64, 64 rows: 169, 269                   FP32, 64: 99, 152
 // and 3x3, which has the FMAs to spare, 128 columns: FP64, 16 rows 118, 160,
-// FP32 82, 84.
-inline bool stepsApply(int size, int H, int nx, int ny)
+// FP32 82, 84.  Such grids are left out where they are most of the batch, but a
+// few beside wider ones cost less in the pass than as three small launches of
+// their own (128 grids of 128 to 2048 points a side, ten steps: 2710 us with them,
+// 2775 without).
+inline bool stepsDouble(int size, int H, int nx)
 {
-    if (nx < 128 || nx >= (1 << 28) || ny < 16) return false;
-    const int single = (nx + 127) / 128;
-    return H == 3 || dev::stepsGrid(size, H, nx, ny, ny).strips < 2 * single;
+    return H == 5 && dev::stepsGrid(size, H, nx, 16, 16).strips >= 2 * ((nx + 127) / 128);
 }
 
 // Several steps in one pass pay once the two sides no longer stay in the L2s
@@ -90,12 +94,18 @@ inline StepsChoice chooseSteps(const std::vector<GridSize>& grids, int size, int
 {
     StepsChoice c;
     c.stepped.assign(grids.size(), 0);
-    int64_t bytes = 0;
+    int64_t bytes = 0, doubled = 0;
     for (size_t i = 0; i < grids.size(); i++) {
         const GridSize& g = grids[i];
-        if (single || !stepsApply(size, H, g.nx, g.ny)) continue;
+        if (single || !stepsApply(g.nx, g.ny)) continue;
         c.stepped[i] = 1;
         bytes += (int64_t)g.nx * g.ny * size;
+        if (stepsDouble(size, H, g.nx)) doubled += (int64_t)g.nx * g.ny * size;
+    }
+    if (doubled > bytes - doubled) {
+        bytes -= doubled;
+        for (size_t i = 0; i < grids.size(); i++)
+            if (stepsDouble(size, H, grids[i].nx)) c.stepped[i] = 0;
     }
     if (bytes <= (H == 5 ? kStepBytes5 : kStepBytes3)) {
         c.stepped.assign(grids.size(), 0);

@@ -4,8 +4,8 @@
  *
  * Many independent periodic xy grids share one stencil (3x3 or 5x5 weights)
  * and are advanced together: each step is one launch over every grid (three
- * steps are, in a batch that outgrows the L2 caches, for the grids at least 16
- * rows high and 128 columns wide, 129 for 5x5), and a run of steps is captured once into a
+ * steps are, in a batch that outgrows the L2 caches, for the grids at least 128
+ * columns wide and 16 rows high), and a run of steps is captured once into a
  * HIP graph.  Per grid the results are
  * bit-identical to cuStenCompute2DXYp followed by cuStenSwap2DXYp.
  */

@@ -45,8 +45,11 @@ def test_a_configured_batch_takes_single_steps(choose, size, H):
 @pytest.mark.parametrize("size", [4, 8])
 def test_grids_whose_strips_double(choose, size):
     """A 5x5 grid of 128 columns takes two strips of a pass, as many points again
-    as a single step computes."""
-    grids = [(400, 128, 300), (80, 129, 300), (80, 256, 300)]
-    assert choose(*grids, size=size, H=5)[1] == [0, 80, 80]
-    assert choose(*grids, size=size, H=3)[1] == [400, 80, 80]
+    as a single step computes: left out where such grids are most of the batch, not
+    where they are few."""
+    wide = [(80, 129, 300), (80, 256, 300)]
+    assert choose((400, 128, 300), *wide, size=size, H=5)[1] == [0, 80, 80]
+    assert choose((200, 128, 300), *wide, size=size, H=5)[1] == [200, 80, 80]
+    assert choose((400, 128, 300), *wide, size=size, H=3)[1] == [400, 80, 80]
     assert choose((1000, 128, 300), size=size, H=5)[1] == [0]
+    assert choose((1000, 128, 300), (1, 256, 300), size=size, H=5)[1] == [0, 0]
