@@ -71,7 +71,11 @@ constexpr int64_t kStepBytes5 = 24 << 20, kStepBytes3 = 16 << 20;
 // length of 128, 64, 32, 16 for which rounds times rows is least, where a wave
 // holds 11 KB of LDS (14 on a CU) and the last round counts 0.4.  In FP32, with
 // twice as many waves on a CU, it takes the longest that gives 12 waves to a
-// CU.  5x5, us per step, by rows:
+// CU.  Waves of lower grids count by their length, and each XCD runs an eighth of
+// the items, in order: where tall grids' long waves would all be on the first
+// XCDs, it is the share of those that counts in FP64, and FP32 takes shorter bands
+// (four 1024 x 1024 grids beside 1000 of 300 x 20: 44 us a step with bands of 128
+// rows, 20 with 32).  5x5, us per step, by rows:
 //   FP64, forty 2048 x 2048 grids     64: 268   128: 262   256: 268
 //   FP64, sixteen 2048 x 2048 grids   64: 115   128: 125
 //   FP64, sixteen 1024 x 1024 grids   16: 41.3   32: 37.5
@@ -79,6 +83,7 @@ constexpr int64_t kStepBytes5 = 24 << 20, kStepBytes3 = 16 << 20;
 //   FP32, 32 1024 x 1024 grids        32: 43.8   64: 37.5
 constexpr int kStepRows = 128;
 constexpr int kStepSlots = 14 * 256, kStepWaves32 = 12 * 256;
+constexpr double kStepUneven = 1.25;  // most work of an XCD against the mean
 
 struct GridSize {
     int nx, ny;
@@ -113,19 +118,40 @@ inline StepsChoice chooseSteps(const std::vector<GridSize>& grids, int size, int
     }
     double least = 0;
     for (int rows = kStepRows; rows >= 16; rows /= 2) {
-        int64_t waves = 0;
+        int64_t items = 0;
         for (size_t i = 0; i < grids.size(); i++) {
             if (!c.stepped[i]) continue;
             const dev::StepsGrid s = dev::stepsGrid(size, H, grids[i].nx, grids[i].ny, rows);
-            waves += (int64_t)s.strips * s.bands;
+            items += (int64_t)s.strips * s.bands;
         }
-        const double time = std::max(1.0, (double)waves / kStepSlots + 0.4) *
-                            (rows + dev::kFusedSteps * (H - 1) + 6);
+        // row-steps of the longest wave and of an XCD's (6: what a wave costs beside)
+        const int64_t share = std::max<int64_t>(1, (items + 7) / 8);
+        double longest = 0, work = 0, most = 0, here = 0;
+        int64_t room = share;
+        for (size_t i = 0; i < grids.size(); i++) {
+            if (!c.stepped[i]) continue;
+            const dev::StepsGrid s = dev::stepsGrid(size, H, grids[i].nx, grids[i].ny, rows);
+            const double wave = std::min(rows, grids[i].ny) + dev::kFusedSteps * (H - 1) + 6;
+            longest = std::max(longest, wave);
+            for (int64_t n = (int64_t)s.strips * s.bands; n > 0;) {
+                const int64_t k = std::min(n, room);
+                work += wave * k;
+                here += wave * k;
+                most = std::max(most, here);
+                n -= k;
+                room -= k;
+                if (room == 0) {
+                    here = 0;
+                    room = share;
+                }
+            }
+        }
+        const double time = std::max(1.0, 8 * most / longest / kStepSlots + 0.4) * longest;
         if (rows == kStepRows || size == 4 || time < least) {
             least = time;
             c.rows = rows;
         }
-        if (size == 4 && waves >= kStepWaves32) break;
+        if (size == 4 && work / longest >= kStepWaves32 && 8 * most <= kStepUneven * work) break;
     }
     return c;
 }

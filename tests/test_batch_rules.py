@@ -53,3 +53,16 @@ def test_grids_whose_strips_double(choose, size):
     assert choose((400, 128, 300), *wide, size=size, H=3)[1] == [400, 80, 80]
     assert choose((1000, 128, 300), size=size, H=5)[1] == [0]
     assert choose((1000, 128, 300), (1, 256, 300), size=size, H=5)[1] == [0, 0]
+
+
+@pytest.mark.parametrize("size,H,grids,rows", [
+    (4, 5, [(16, 1024, 1024)], 32), (4, 5, [(32, 1024, 1024)], 64), (4, 5, [(16, 2048, 2048)], 128),
+    (8, 5, [(16, 1024, 1024)], 32), (8, 5, [(16, 2048, 2048)], 64), (8, 5, [(40, 2048, 2048)], 128),
+    # tall grids beside low ones, whose waves are short
+    (4, 5, [(4, 1024, 1024), (1000, 300, 20)], 32), (4, 3, [(7, 1024, 1024), (3000, 128, 20)], 32),
+    (4, 5, [(7, 1024, 1024), (3500, 128, 16)], 16), (4, 3, [(1, 2048, 2048), (8000, 130, 20)], 32),
+])
+def test_rows_of_bands(choose, size, H, grids, rows):
+    """Bands of the length that was measured as the fastest; in FP32 low grids' many
+    short waves do not stand for tall grids' few long ones."""
+    assert choose(*grids, size=size, H=H)[0] == rows
