@@ -389,6 +389,13 @@ constexpr int kDefaultRPW = 8;
 constexpr int kDefaultChunks = 4;
 // From this many points on, bands of 8 rows still make 8 waves per CU.
 constexpr int64_t kLongBandPoints = int64_t(1) << 21;
+// The 1x13 walker's bands of 8 rows read 20; bands of 12 read 24, with a third
+// fewer waves.  From this many points on that is never the worse exchange:
+//   us, 8 rows against 12: 8192^2 FP32 90, 80 (chunked strips: 87)   FP64 182, 172
+//   4096^2 FP32 25.0, 24.0   FP64 42.4, 42.0   2048^2 FP32 9.6, 8.6   FP64 13.5, 13.0
+//   2048 x 1500 FP32 7.5, 7.4   FP64 8.9, 10.3
+// 1x11 keeps 8 rows: 12 lose on most grids (FP32 7001 x 6001: 50 us, 53.5).
+constexpr int64_t kTallBandPoints = int64_t(1) << 22;
 
 template <typename T>
 bool pairAligned(const void* p, int64_t ld)
@@ -613,7 +620,11 @@ hipError_t launchStencil(const StencilLaunch& in, hipStream_t st, KernelUse* use
         s.chunks = s.xform == Xform::Identity
                        ? stencilRowsChunks(s.dtype, s.H, s.V, s.nx, s.ny)
                        : 0;
-        if (s.chunks == 0) s.chunks = (int64_t)s.nx * s.ny >= kLongBandPoints ? 2 : 1;
+        const int64_t points = (int64_t)s.nx * s.ny;
+        if (s.chunks == 0)
+            s.chunks = s.H == 1 && s.V == 13 && points >= kTallBandPoints ? 3
+                       : points >= kLongBandPoints                        ? 2
+                                                                          : 1;
     }
     if (s.colsPerLane != 1) s.colsPerLane = 2;
     if (s.colsPerLane == 1) {
